@@ -15,7 +15,7 @@
 #include "../../include/galx.h"
 #include "galx_adjoint.hpp"
 #include "galx_kernels.hpp"
-#include "galx_kernels_ho.hpp"
+#include "galx_kernels_plane.hpp"
 
 using namespace galx;
 
@@ -248,7 +248,7 @@ __global__ void __launch_bounds__(256) k_pressure_sum(long nDOF, int n3, double 
 struct KernelSet {
     bool ok = false;
     int block = 0;
-    size_t ws_per_elem = 0;  // bytes of workspace per element (the high-order kernels, N >= 10)
+    size_t (*ws_bytes)(int) = nullptr;  // workspace of a mesh of that many elements (the plane kernels)
     void (*trace)(hipStream_t, int, const double*, Mesh, void*, GasD) = nullptr;
     void (*lift)(hipStream_t, int, const double*, Mesh, const void*, void*, const void*, GasD, double, double) = nullptr;
     void (*rhs)(hipStream_t, int, const double*, double*, Mesh, const void*, const void*, void*, double*, double*,
@@ -264,6 +264,10 @@ struct KernelSet {
 template <int N, typename T, bool SPLIT>
 struct Launch {
     using D = Dm<N>;
+    // has the degree kernels with one element per workgroup, and plane kernels
+    static constexpr bool whole = N < GALX_PLANE_DEGREE, planes = use_planes<N, T>(1);
+    static dim3 plane_grid(int nE) { return dim3(8 * plane_per_xcd(nE * Pl<N>::groups)); }
+    static size_t ws_bytes(int nE) { return use_planes<N, T>(nE) ? (size_t)nE * Pl<N>::ws * sizeof(T) : 0; }
     static void trace(hipStream_t s, int nE, const double* U, Mesh m, void* utr, GasD g)
     {
         hipLaunchKernelGGL((k_trace<N, T>), dim3(nE), dim3(D::block), 0, s, U, m, (T*)utr, g);
@@ -271,11 +275,14 @@ struct Launch {
     static void lift(hipStream_t s, int nE, const double* U, Mesh m, const void* utr, void* vtr, const void* mats,
                      GasD g, double LHm, double LHp)
     {
-        if constexpr (D::node_per_thread)
+        if constexpr (planes)
+            if (use_planes<N, T>(nE)) {
+                hipLaunchKernelGGL((k_vol_plane<N, T, T, SPLIT>), plane_grid(nE), dim3(Pl<N>::block), 0, s, nE, U, m,
+                                   (const T*)utr, (T*)vtr, (const T*)mats, g, T(LHm), T(LHp));
+                return;
+            }
+        if constexpr (whole)
             hipLaunchKernelGGL((k_lift<N, T, T>), dim3(nE), dim3(D::block), 0, s, U, m, (const T*)utr, (T*)vtr,
-                               (const T*)mats, g, T(LHm), T(LHp));
-        else
-            hipLaunchKernelGGL((k_lift_ho<N, T, T>), dim3(nE), dim3(D::block), 0, s, U, m, (const T*)utr, (T*)vtr,
                                (const T*)mats, g, T(LHm), T(LHp));
     }
     template <int RIE>
@@ -283,12 +290,15 @@ struct Launch {
                       void* utr_next, double* Ut, double* K, const void* mats, GasD g, double LHm, double LHp,
                       Stage st)
     {
-        if constexpr (D::node_per_thread)
+        if constexpr (planes)
+            if (use_planes<N, T>(nE)) {
+                hipLaunchKernelGGL((k_upd_plane<N, T, T, SPLIT, RIE>), plane_grid(nE), dim3(Pl<N>::block), 0, s, nE, U,
+                                   Uout, m, (const T*)utr, (const T*)vtr, (T*)utr_next, Ut, K, (const T*)mats, g,
+                                   T(LHm), T(LHp), st);
+                return;
+            }
+        if constexpr (whole)
             hipLaunchKernelGGL((k_rhs<N, T, T, SPLIT, RIE>), dim3(nE), dim3(D::block), 0, s, U, Uout, m,
-                               (const T*)utr, (const T*)vtr, (T*)utr_next, Ut, K, (const T*)mats, g, T(LHm), T(LHp),
-                               st);
-        else
-            hipLaunchKernelGGL((k_rhs_ho<N, T, T, SPLIT, RIE>), dim3(nE), dim3(D::block), 0, s, U, Uout, m,
                                (const T*)utr, (const T*)vtr, (T*)utr_next, Ut, K, (const T*)mats, g, T(LHm), T(LHp),
                                st);
     }
@@ -312,11 +322,11 @@ struct Launch {
     static void grad(hipStream_t s, int nE, const double* U, Mesh m, const void* utr, const void* mats, GasD g,
                      double LHm, double LHp, double* gvol)
     {
-        if constexpr (D::node_per_thread)
-            hipLaunchKernelGGL((k_grad<N, T, T>), dim3(nE), dim3(D::block), 0, s, U, m, (const T*)utr,
-                               (const T*)mats, g, T(LHm), T(LHp), gvol);
+        if constexpr (!whole)
+            hipLaunchKernelGGL((k_grad_plane<N, T, T>), plane_grid(nE), dim3(Pl<N>::block), 0, s, nE, U, m,
+                               (const T*)utr, (const T*)mats, g, T(LHm), T(LHp), gvol);
         else
-            hipLaunchKernelGGL((k_grad_ho<N, T, T>), dim3(nE), dim3(D::block), 0, s, U, m, (const T*)utr,
+            hipLaunchKernelGGL((k_grad<N, T, T>), dim3(nE), dim3(D::block), 0, s, U, m, (const T*)utr,
                                (const T*)mats, g, T(LHm), T(LHp), gvol);
     }
     static void grad_rho(hipStream_t s, int nE, const double* U, Mesh m, const void* utr, const double* DT64,
@@ -332,7 +342,7 @@ struct Launch {
         k.grad_rho = &grad_rho;
         k.ok = true;
         k.block = D::block;
-        k.ws_per_elem = D::node_per_thread ? 0 : HoWs<N>::size * sizeof(T);
+        k.ws_bytes = &ws_bytes;
         k.trace = &trace;
         k.lift = &lift;
         k.rhs = &rhs;
@@ -449,7 +459,7 @@ struct galx_ctx {
     double *dU = nullptr, *dK = nullptr, *dUt = nullptr, *dScratch = nullptr;
     double *dGeo = nullptr, *dFgeo = nullptr, *dSgeo = nullptr;
     float *dGeo32 = nullptr, *dFgeo32 = nullptr, *dSgeo32 = nullptr;  // mixed form: FP32 roundings of the three
-    void* dWs = nullptr;  // per-element workspace of the high-order kernels (N >= 10)
+    void* dWs = nullptr;  // per-element workspace of the plane kernels
     int *dConn = nullptr, *dInv = nullptr;
     void *dUtr[2] = {nullptr, nullptr}, *dVtr = nullptr, *dMats = nullptr;
     double *dDtc = nullptr, *dDtv = nullptr, *dDtOut = nullptr;
@@ -641,7 +651,8 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
     if ((rc = dalloc(c, &c->dK, 5 * nDOF * sizeof(double)))) return rc;
     if ((rc = dalloc(c, &c->dGeo, 10 * nDOF * sizeof(double)))) return rc;
     if ((rc = dalloc(c, &c->dFgeo, 10 * nfn * sizeof(double)))) return rc;
-    const int ns = surface_count(c->cfg.N);
+    // the surface-node copy of the geometry is k_lift's
+    const int ns = c->N < GALX_PLANE_DEGREE ? surface_count(c->N) : 0;
     if ((rc = dalloc(c, &c->dSgeo, 10L * nElems * ns * sizeof(double)))) return rc;
     if ((rc = dalloc(c, &c->dConn, 6L * nElems * sizeof(int)))) return rc;
     if ((rc = dalloc(c, &c->dInv, inv.size() * sizeof(int)))) return rc;
@@ -652,7 +663,7 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
     if ((rc = dalloc(c, &c->dDtv, nElems * sizeof(double)))) return rc;
     if ((rc = dalloc(c, &c->dDtOut, 4 * sizeof(double)))) return rc;
     if ((rc = dalloc(c, &c->dErr, sizeof(int)))) return rc;
-    if (c->ks.ws_per_elem && (rc = dalloc(c, (char**)&c->dWs, c->ks.ws_per_elem * nElems))) return rc;
+    if (const size_t b = c->ks.ws_bytes(nElems); b && (rc = dalloc(c, (char**)&c->dWs, b))) return rc;
     if (c->tsz == 4) {
         if ((rc = dalloc(c, &c->dGeo32, 10 * nDOF * sizeof(float)))) return rc;
         if ((rc = dalloc(c, &c->dFgeo32, 10 * nfn * sizeof(float)))) return rc;
@@ -668,7 +679,7 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
     Staging stg;
     if ((rc = stg.init(stageB))) return rc;
     std::vector<int> snode(ns);
-    for (int t = 0; t < ns; t++) snode[t] = surface_node_of(c->cfg.N, t);
+    for (int t = 0; t < ns; t++) snode[t] = surface_node_of(c->N, t);
     for (long e0 = 0; e0 < nElems; e0 += chunkE) {
         long ne = std::min(chunkE, (long)nElems - e0);
         double* buf = stg.next();
@@ -692,8 +703,9 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
         }
         HIPCHK(hipMemcpyAsync(c->dGeo + e0 * 10 * n3, buf, ne * 10 * n3 * sizeof(double), hipMemcpyHostToDevice,
                               c->stream));
-        HIPCHK(hipMemcpyAsync(c->dSgeo + e0 * 10 * ns, sbuf, ne * 10 * ns * sizeof(double), hipMemcpyHostToDevice,
-                              c->stream));
+        if (ns)
+            HIPCHK(hipMemcpyAsync(c->dSgeo + e0 * 10 * ns, sbuf, ne * 10 * ns * sizeof(double), hipMemcpyHostToDevice,
+                                  c->stream));
         if ((rc = stg.issued(c->stream))) return rc;
     }
     for (long s0 = 0; s0 < nSides; s0 += chunkS) {
@@ -722,8 +734,9 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
                                                         {c->dSgeo, c->dSgeo32}};
         const long len[3] = {10 * nDOF, 10 * nfn, 10L * nElems * ns};
         for (int a = 0; a < 3; a++)
-            k_round_f32<<<dim3((unsigned)((len[a] + 255) / 256)), dim3(256), 0, c->stream>>>(len[a], cp[a].first,
-                                                                                           cp[a].second);
+            if (len[a])
+                k_round_f32<<<dim3((unsigned)((len[a] + 255) / 256)), dim3(256), 0, c->stream>>>(len[a], cp[a].first,
+                                                                                               cp[a].second);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(c->stream));

@@ -34,7 +34,8 @@
 namespace galx {
 
 // one workgroup per element: n^3 threads rounded up to whole waves, at most 1024 (N <= 9 gives every volume node a
-// thread of its own; the high-order kernels of N >= 10 loop their 1024 threads over the nodes)
+// thread of its own; for N >= 10 the plane kernels take the stage, and the kernels here that run for every degree loop
+// their 1024 threads over the nodes)
 template <int N>
 struct Dm {
     static constexpr int n = N + 1, n2 = n * n, n3 = n2 * n, nf = 6 * n2;
@@ -165,7 +166,7 @@ struct Mesh {
     const float* geo32;
     const float* fgeo32;
     const float* sgeo32;
-    void* ws;  // per-element workspace of the high-order kernels (N >= 10), else null
+    void* ws;  // per-element workspace of the plane kernels, else null
 };
 
 // the geometry arrays a kernel of compute type T reads its metric and face operands from

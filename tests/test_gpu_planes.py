@@ -1,0 +1,70 @@
+"""GPU parity on both sides of the line between the stage kernels that take one element per workgroup and those that
+split it into k-planes (use_planes in galx_kernels_plane.hpp: FP64, 4 <= N <= 9, at most 1024 planes in the mesh), on
+meshes with uneven sides, curved and with rotated elements: Ut and one LSERK step against the FP64 oracle.
+
+Bar: the FP64 bar of the parity tests, 1e-12 relative L2, plus four times what a change of U by one unit in the last
+place does to the oracle's own result.  On meshes with many elements along one direction that is the larger part: the
+viscous terms amplify rounding with the square of their number while Ut of the smooth state stays the same size (5.8e-12
+for 43 elements at N = 7, where the one-element kernels are 3.9e-12 from the oracle)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from galaexi_amd import mesh as M
+from galaexi_amd import testcases as T
+
+pytestmark = pytest.mark.gpu
+
+RIE = {"lf": O.RIEMANN_LF, "roe": O.RIEMANN_ROE, "roeentropyfix": O.RIEMANN_ROEEF}
+BELOW = {4: (17, 4, 3), 5: (17, 5, 2), 6: (9, 4, 4), 7: (8, 4, 4), 8: (7, 4, 4), 9: (17, 3, 2)}
+ABOVE = {4: (7, 6, 5), 5: (9, 19, 1), 6: (7, 7, 3), 7: (43, 3, 1), 8: (19, 3, 2), 9: (103, 1, 1)}
+FORMS = {4: ("split", "roe"), 5: ("weak", "roeentropyfix"), 6: ("split", "lf"), 7: ("split", "roeentropyfix"),
+         8: ("weak", "lf"), 9: ("split", "lf")}
+
+
+def planes(nel, N):
+    return int(np.prod(nel)) * (N + 1)
+
+
+def test_sizes_lie_on_their_side_of_the_line():
+    assert all(planes(nel, N) <= 1024 for N, nel in BELOW.items())
+    assert all(planes(nel, N) > 1024 for N, nel in ABOVE.items())
+
+
+@pytest.mark.parametrize("side", ["below", "above"])
+@pytest.mark.parametrize("N", sorted(FORMS))
+def test_stage_kernels_vs_oracle(N, side):
+    from galaexi_amd import dg
+
+    form, riemann = FORMS[N]
+    nel = (BELOW if side == "below" else ABOVE)[N]
+    print(f"case: N={N} {nel} {form} {riemann}", flush=True)
+    lo, hi = (-1.0, -1.0, -1.0), (1.0, 1.0, 1.0)
+    m = M.box_mesh(nel, N, lo=lo, hi=hi, deform_amp=0.03, deform_phase=(0.13, 0.37, 0.71), NGeo=2,
+                   rotations="random" if min(nel) > 1 else None, seed=N)
+    U = T.smooth_random(m.Elem_xGP, lo, hi, seed=N, kmax=1)
+    gas = dict(mu0=2e-2, R=1.0, Pr=0.72, kappa=1.4)
+    op = dg.DGOperator(N, form=form, riemann=riemann, **gas)
+    op.set_mesh(m)
+    op.set_state(U)
+    ref = O.Operator(m, split=form == "split", riemann=RIE[riemann], **gas)
+    ulp = np.random.default_rng(0).choice([-1.0, 1.0], U.shape) * np.finfo(float).eps
+    U1 = np.asfortranarray(U * (1.0 + ulp))
+
+    def check(got, want, want1, scale, what):
+        err, own = (np.linalg.norm((a - want).ravel()) for a in (got, want1))
+        assert err <= 1e-12 * np.linalg.norm(scale.ravel()) + 4.0 * own, (what, err, own, np.linalg.norm(scale.ravel()))
+
+    Ut, Ur, Ur1 = op.DGTimeDerivative_weakForm(0.0), ref.rhs(U), ref.rhs(U1)
+    for v in range(5):
+        check(Ut[v], Ur[v], Ur1[v], Ur[v], v)
+    dt, errType = op.CalcTimeStep()
+    assert errType == 0
+    op.TimeStepByLSERKW2(0.0, dt)
+    Ug = op.get_state()
+    op.close()
+    W = []
+    for start in (U, U1):
+        W.append(np.asfortranarray(start.copy()))
+        ref.lserk_step(W[-1], np.zeros_like(U, order="F"), 0.0, dt)
+    check(Ug, W[0], W[1], W[0] - U, "step")
