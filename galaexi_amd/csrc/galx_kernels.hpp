@@ -392,22 +392,12 @@ __device__ __forceinline__ void gradient_combine(int node, const T* s_lflux, T L
     }
 }
 
-// the same with fewer live registers (k_lift): each direction's derivatives become the Cartesian sums as they are
-// formed, and the surface terms are added to those sums face by face, with no separate surface accumulator.  The
-// sums round in another order than gradient_combine's, within the FP64 parity bar.
+// the surface terms of the lean gradient and the scaling with sJ
 template <int N, typename T>
-__device__ __forceinline__ void gradient_combine_lean(int node, const T* s_lflux, T LHm, T LHp, const T* gm, T* gxi,
-                                                      T* get, T* gze, T* g)
+__device__ __forceinline__ void gradient_surface_lean(int node, const T* s_lflux, T LHm, T LHp, T sJ, T* g)
 {
     constexpr int n = N + 1, n2 = n * n;
     const int i = node % n, j = (node / n) % n, k = node / n2;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const T a = gxi[q], b = get[q], c = gze[q];
-        g[q] = gm[0] * a + gm[3] * b + gm[6] * c;
-        g[4 + q] = gm[1] * a + gm[4] * b + gm[7] * c;
-        g[8 + q] = gm[2] * a + gm[5] * b + gm[8] * c;
-    }
 #pragma unroll
     for (int ls = 1; ls <= 6; ls++) {
         int ab;
@@ -423,14 +413,30 @@ __device__ __forceinline__ void gradient_combine_lean(int node, const T* s_lflux
             g[8 + q] = g[8 + q] + (lf * n2v) * LH;
         }
     }
-    const T sJ = gm[9];
 #pragma unroll
     for (int q = 0; q < 12; q++) g[q] = sJ * g[q];
 }
 
+// the same with fewer live registers: each direction's derivatives become the Cartesian sums as they are
+// formed, and the surface terms are added to those sums face by face, with no separate surface accumulator.  The
+// sums round in another order than gradient_combine's, within the FP64 parity bar.
+template <int N, typename T>
+__device__ __forceinline__ void gradient_combine_lean(int node, const T* s_lflux, T LHm, T LHp, const T* gm, T* gxi,
+                                                      T* get, T* gze, T* g)
+{
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const T a = gxi[q], b = get[q], c = gze[q];
+        g[q] = gm[0] * a + gm[3] * b + gm[6] * c;
+        g[4 + q] = gm[1] * a + gm[4] * b + gm[7] * c;
+        g[8 + q] = gm[2] * a + gm[5] * b + gm[8] * c;
+    }
+    gradient_surface_lean<N, T>(node, s_lflux, LHm, LHp, gm[9], g);
+}
+
 // gm: the node's Ja^1(3), Ja^2(3), Ja^3(3), sJ (load_node_geo), loaded by the caller ahead of the barrier that
 // precedes this call so that their latency overlaps the face tasks.  LEAN: the line loop one step at a time and
-// gradient_combine_lean, so that k_lift fits 80 registers without spilling (three FP64 workgroups per CU)
+// gradient_combine_lean, so that k_lift fits 80 registers without spilling (three FP64 workgroups per CU at N = 7)
 template <int N, typename T, class MT, bool LEAN = false>
 __device__ __forceinline__ void node_gradient(int node, const MT& M, const T* s_lift, const T* s_lflux,
                                               T LHm, T LHp, const T* gm, T* g)
@@ -459,6 +465,45 @@ __device__ __forceinline__ void node_gradient(int node, const MT& M, const T* s_
         gradient_combine_lean<N, T>(node, s_lflux, LHm, LHp, gm, gxi, get, gze, g);
     else
         gradient_combine<N, T>(node, s_lflux, LHm, LHp, gm, gxi, get, gze, g);
+}
+
+// the lean gradient with one direction after the other: 4 instead of 12 accumulators live in the line loops.  For FP64
+// degrees whose lines are not powers of two long: k_lift 4 to 14 % faster for N = 6, 8 and 9 on MI355X (75 -> 67
+// registers).  At N = 7, whose 64-byte line strides meet in the LDS banks, the interleaved directions of the plain loop
+// measured 2 % faster in k_rhs; up to N = 4 the three short loops cost what they save.  The mixed form keeps the plain
+// loop and with it its FP32 rounding.
+template <int N, typename T>
+__host__ __device__ constexpr bool gradient_in_sequence()
+{
+    return sizeof(T) == 8 && N >= 5 && ((N + 1) & N) != 0;
+}
+
+template <int N, typename T, class MT>
+__device__ __forceinline__ void node_gradient_seq(int node, const MT& M, const T* s_lift, const T* s_lflux, T LHm,
+                                                  T LHp, const T* gm, T* g)
+{
+    constexpr int n = N + 1, n2 = n * n;
+    constexpr int n3p = Lay<N>::n3;
+    const int i = node % n, j = (node / n) % n, k = node / n2;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int idx = d == 0 ? i : (d == 1 ? j : k);
+        const auto ln = Lay<N>::line(d, i, j, k);
+        T a[4] = {0, 0, 0, 0};
+#pragma unroll 1
+        for (int l = 0; l <= N; l++) {
+            const T dl = M.dt(l, idx);
+            const int o = ln(l);
+#pragma unroll
+            for (int q = 0; q < 4; q++) a[q] = a[q] + dl * s_lift[q * n3p + o];
+        }
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                g[4 * c + q] = d == 0 ? gm[c] * a[q] : g[4 * c + q] + gm[3 * d + c] * a[q];
+    }
+    gradient_surface_lean<N, T>(node, s_lflux, LHm, LHp, gm[9], g);
 }
 
 // 16x16x4 matrix-core step of type T: D = A B + C with A 16x4, B 4x16; lane l holds A[l % 16][l / 16] and
@@ -592,17 +637,11 @@ __host__ __device__ __forceinline__ int surface_node(int t)
 template <int N, typename T, typename TT, bool TR>
 __device__ __forceinline__ void lift_gradient(int e, int tid, const Mesh& mesh, const TT* __restrict__ utr,
                                               const Mats<N, T, TR>& M, const T* s_lift, T* s_lflux,
-                                              const Gas<T>& gas, T LHm, T LHp, T* g, T* s_nb = nullptr,
-                                              const T* gm = nullptr)
+                                              const Gas<T>& gas, T LHm, T LHp, T* g)
 {
-    lift_face_fluxes<N, T, TT>(e, tid, mesh, utr, s_lift, s_lflux, gas, s_nb);
+    lift_face_fluxes<N, T, TT>(e, tid, mesh, utr, s_lift, s_lflux, gas, nullptr);
     __syncthreads();
-    if (tid < Dm<N>::n3) {
-        if (gm)
-            node_gradient<N, T>(tid, M, s_lift, s_lflux, LHm, LHp, gm, g);
-        else
-            node_gradient<N, T, TR>(e, tid, mesh, M, s_lift, s_lflux, LHm, LHp, g);
-    }
+    if (tid < Dm<N>::n3) node_gradient<N, T, TR>(e, tid, mesh, M, s_lift, s_lflux, LHm, LHp, g);
 }
 
 // volume state of node tid: ConsToPrim (eos.f90:212-239) in FP64, then shifted by the pressure offset and
@@ -734,7 +773,12 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     T g[12];
     lift_face_fluxes<N, T, TT>(e, tid, mesh, utr, s_lift, s_lflux, gas, nullptr);
     __syncthreads();
-    if (gnode) node_gradient<N, T, MatsD<N, T>, true>(gn, M, s_lift, s_lflux, LHm, LHp, gm, g);
+    if (gnode) {
+        if constexpr (gradient_in_sequence<N, T>())
+            node_gradient_seq<N, T>(gn, M, s_lift, s_lflux, LHm, LHp, gm, g);
+        else
+            node_gradient<N, T, MatsD<N, T>, true>(gn, M, s_lift, s_lflux, LHm, LHp, gm, g);
+    }
     __syncthreads();
     // the stress tensor and heat flux of each surface node (the terms of EvalNormalDiffFlux3D, flux.f90:779-847,
     // before the normal) to its face slots: 9 values per face node instead of the 12 gradients (9 KB less LDS at
@@ -880,8 +924,31 @@ __global__ void __launch_bounds__(Dm<N>::block)
 // U is read and the new state written to Uout, which may be U itself (in-place LSERK update) or another
 // buffer (the adjoint's recompute keeps every stage input).
 // ---------------------------------------------------------------------------------------------------------
-template <int N, typename T, typename TT, bool SPLIT, int RIEMANN>
-__device__ __forceinline__ void face_flux(const T* tro, const T* fvo, const T* trn, const T* fvn,
+// The lean order of the FP64 form, for fewer live registers and less LDS: the lean gradient; in the split form the viscous
+// terms of all directions before the pairs (the stress tensor dies before the pairs, whose sum then starts from the
+// viscous one, and 9 instead of 13 node planes share the work region); the viscous-flux traces loaded after the Riemann
+// flux.  Registers without a cap at N = 7 (split): LF 126 (capped, 128) -> 102, Roe 150 -> 116, RoeEntropyFix 142 -> 120,
+// so that every solver runs two 8-wave workgroups per CU without spilling; LDS at N = 7 71.7 -> 55.3, at N = 8
+// 97 -> 74 KB (two workgroups per CU).  k_rhs on MI355X, FP64, before -> after:
+//   split RoeEntropyFix N = 7, 20^3 elements   645 -> 443 us     split LF N = 8, 16^3   441 -> 344 us
+//   split LF N = 6, 16^3                       201 -> 182 us     split LF N = 5, 24^3   315 -> 303 us
+//   weak Roe N = 5, 20^3                       220 -> 187 us
+// Split LF at N = 7 keeps the other order, with the lifting's line derivatives on the matrix cores (node_gradient_mfma,
+// no registers to spare for Roe beside it): it runs at two workgroups per CU either way, and the stage, the k_lift behind
+// it included, measured 0.5 to 0.8 % faster.
+// For smaller elements, one or two waves each, the order that keeps more in flight is as fast or faster (split LF N = 4
+// 118 against 123 us on 20^3, N = 3 weak Roe 111 against 116 us on 24^3).  The mixed form, which fits three workgroups
+// per CU as it is, runs 2 % slower in the lean order and keeps its own, and with it its FP32 rounding.
+template <int N, typename T, bool SPLIT, int RIEMANN>
+__host__ __device__ constexpr bool rhs_lean()
+{
+    return sizeof(T) == 8 && N >= (SPLIT ? 5 : 4) && !(N == 7 && SPLIT && RIEMANN == RIEMANN_LF);
+}
+
+// numerical flux F times SurfElem of a face node from both sides' trace records (tro own, trn neighbour) and viscous-flux
+// traces: values fv[8] (own, neighbour), with LATE loaded here from fvo and fvn
+template <int N, typename T, typename TT, bool SPLIT, int RIEMANN, bool LATE>
+__device__ __forceinline__ void face_flux(const T* tro, const T* trn, T* fv, const TT* fvo, const TT* fvn,
                                           const T* __restrict__ fg, int n2, int flip, const Gas<T>& gas, T* F)
 {
     T Uo[5], Un[5], Po[6], Pn[6];
@@ -897,24 +964,40 @@ __device__ __forceinline__ void face_flux(const T* tro, const T* fvo, const T* t
         T t2[3] = {fg[6 * n2], fg[7 * n2], fg[8 * n2]};
         riemann_point<T, SPLIT>(RIEMANN, UL, UR, PL, PR, nv, t1, t2, gas, F);
     }
+    if (LATE) {
+        // the viscous-flux traces, behind the Riemann flux: the scheduler would move the loads up again, 16 registers
+        // held through the solver
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            fv[v] = T(fvo[v * n2]);
+            fv[4 + v] = T(fvn[v * n2]);
+        }
+    }
     // ViscousFlux (riemann.f90:638-700): 0.5*(F_v(master) + F_v(slave)).n, summed in an order both sides share
     T se = fg[9 * n2];
     F[0] = F[0] * se;
 #pragma unroll
-    for (int v = 1; v < 5; v++) F[v] = (F[v] + (T(0.5) * fvo[v - 1] + T(0.5) * fvn[v - 1])) * se;
+    for (int v = 1; v < 5; v++) F[v] = (F[v] + (T(0.5) * fv[v - 1] + T(0.5) * fv[3 + v])) * se;
 }
 
-// minimum waves per SIMD for k_rhs: 4 lets two 512-thread workgroups share a CU at N=7 in FP64 (registers capped
-// at 128), 6 lets three share it in the mixed form (capped at 80, which its LDS share allows); the heavier
-// entropy-fixed Roe solver and the small blocks of N<5 keep the compiler's choice.
-template <int N, int RIEMANN, typename T>
+// minimum waves per SIMD for k_rhs.  FP64: the compiler's choice (at most 128 registers in the lean order) except where
+// LF, the lightest solver, fits one workgroup more without spilling or with little of it: 5 waves at N = 5 (five 4-wave
+// workgroups per CU, 99 against 103 us on 16^3 elements) and at N = 6 in the split form (three 6-wave ones), 6 at N = 8 in
+// the split form (two 12-wave ones, 80 registers with 6 spilled: 344 against 445 us on 16^3).  The Roe solvers spill
+// under the same caps and lose (N = 6 Roe 218 -> 251 us).  Mixed: 6 lets three 512-thread workgroups share a CU at N = 7
+// (80 registers, which its LDS share allows); the entropy-fixed Roe solver and the small blocks of N < 5 keep the
+// compiler's choice.
+template <int N, int RIEMANN, typename T, bool SPLIT>
 struct RhsWaves {
+    static constexpr int fp64 =
+        RIEMANN != RIEMANN_LF ? 1 : (N == 5 || (N == 6 && SPLIT) ? 5 : (N == 8 && SPLIT ? 6 : 1));
     static constexpr int value =
-        (RIEMANN == RIEMANN_ROEEF || Dm<N>::block < 256) ? 1 : (sizeof(T) == 4 ? GALX_MIXED_WAVES : 4);
+        sizeof(T) == 8 ? fp64 : (RIEMANN == RIEMANN_ROEEF || Dm<N>::block < 256 ? 1 : GALX_MIXED_WAVES);
 };
 
 template <int N, typename T, typename TT, bool SPLIT, int RIEMANN>
-__global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T>::value))
+__global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>::value))
     k_rhs(const double* U, double* Uout, Mesh mesh, const TT* __restrict__ utr, const TT* __restrict__ vtr,
           TT* __restrict__ utr_next, double* __restrict__ Ut, double* __restrict__ Kreg, const T* __restrict__ mats,
           GasD gd, T LHm, T LHp, Stage st)
@@ -923,16 +1006,18 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T>::value)
     static_assert(D::node_per_thread, "one volume node per thread: N <= 9");
     constexpr int n = D::n, n2 = D::n2, n3 = D::n3;
     constexpr int np = Lay<N>::np, n3p = Lay<N>::n3;  // padded node layout of the line-read arrays
-    // FP64 at N = 7: the lifting's in-plane line derivatives on the matrix cores (node_gradient_mfma), with a 4 x 64
-    // scratch per wave after the lifting arrays.  The mixed form keeps them on the VALU: with the scratch (6.6 KB more
-    // LDS) it measured 12 % slower on MI355X.
-    constexpr bool mfma_lift = N == 7 && sizeof(T) == 8;
+    constexpr bool lean = rhs_lean<N, T, SPLIT, RIEMANN>();
+    // FP64 at N = 7 in the other order: the lifting's in-plane line derivatives on the matrix cores
+    // (node_gradient_mfma), with a 4 x 64 scratch per wave after the lifting arrays.  The mixed form keeps them on the
+    // VALU: with the scratch (6.6 KB more LDS) it measured 12 % slower on MI355X.
+    constexpr bool mfma_lift = N == 7 && sizeof(T) == 8 && !lean;
     constexpr int w_a0 = 4 * n3p + 6 * 7 * n2;
     constexpr int w_a = w_a0 + (mfma_lift ? 8 * 4 * n2 : 0);  // lifting
     // mixed split form: the nine metric terms of every node stay in LDS (FP32, halves) in s_geo for the whole
     // kernel, so the volume terms read them there instead of from memory a second time (7.8 % faster at N=7)
     constexpr bool geo_lds = SPLIT && sizeof(T) == 4;
-    constexpr int w_c = SPLIT ? (geo_lds ? 10 : 13) * n3p : 5 * n3p;  // volume fluxes / split-form partner data
+    constexpr bool visc_first = SPLIT && lean;
+    constexpr int w_c = SPLIT ? (visc_first ? 9 : (geo_lds ? 10 : 13)) * n3p : 5 * n3p;  // volume terms
     constexpr int w_d = 6 * 5 * n2;  // face results, new traces
     // split form: the i- and j-lines lie inside one 64-lane wave (n and n^2 divide 64: N = 1, 3, 7), so the pairs of
     // those lines are shared between lanes instead of formed twice
@@ -978,16 +1063,18 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T>::value)
     Stress<T> s;
     {
         T g[12];
-        if (mfma_lift) {
-            lift_face_fluxes<N, T, TT>(e, tid, mesh, utr, s_w, s_w + 4 * n3p, gas, s_nb);
+        lift_face_fluxes<N, T, TT>(e, tid, mesh, utr, s_w, s_w + 4 * n3p, gas, s_nb);
+        __syncthreads();
+        if (active) {
             if (!pgeo) load_node_geo<N, T>(e, tid, mesh, gm);
-            __syncthreads();
-            node_gradient_mfma<T>(tid, M, s_w, s_w + 4 * n3p, s_w + w_a0, LHm, LHp, gm, g);
-        } else {
-            lift_gradient<N, T, TT>(e, tid, mesh, utr, M, s_w, s_w + 4 * n3p, gas, LHm, LHp, g, s_nb,
-                                    pgeo ? gm : nullptr);
+            if constexpr (mfma_lift)
+                node_gradient_mfma<T>(tid, M, s_w, s_w + 4 * n3p, s_w + w_a0, LHm, LHp, gm, g);
+            else if constexpr (gradient_in_sequence<N, T>())
+                node_gradient_seq<N, T>(tid, M, s_w, s_w + 4 * n3p, LHm, LHp, gm, g);
+            else
+                node_gradient<N, T, Mats<N, T>, lean>(tid, M, s_w, s_w + 4 * n3p, LHm, LHp, gm, g);
+            stress(pr, g, gas, s);
         }
-        if (active) stress(pr, g, gas, s);
     }
     __syncthreads();
 
@@ -1021,119 +1108,165 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T>::value)
             line_sync<N>(d);
         }
     } else {
-        // ---- per direction: viscous contravariant flux with the weak-form D_Hat_T contraction
-        // (VolInt_weakForm_Visc) and the split-form flux differencing (VolInt_splitForm_Kernel); the direction's
-        // metric is read once for both ----
+        // ---- viscous contravariant flux with the weak-form D_Hat_T contraction (VolInt_weakForm_Visc) and split-form
+        // flux differencing (VolInt_splitForm_Kernel) ----
         // the split flux runs on halves (split_volume_flux_pi_half): s_v and s_m hold half of each node's
         // (rho,u,v,w,p,H) and metric, and the sum is doubled once at the end (exact)
-        T* s_v = s_w;                                // [6][n3p] rho,u,v,w,p,H (halves)
-        T* s_m = s_w + 6 * n3p;                      // [3][n3p] metric of the current direction (halves)
-        T* s_f = s_w + (geo_lds ? 6 : 9) * n3p;      // [4][n3p] viscous contravariant flux (momentum, energy) of
-                                                     // the current direction
+        T* s_v = s_w;  // [6][n3p] rho,u,v,w,p,H (halves)
         const T hv[6] = {T(0.5) * pr[0], T(0.5) * pr[1], T(0.5) * pr[2], T(0.5) * pr[3], T(0.5) * pr[4],
                          T(0.5) * Hme};
-        if (active) {
-#pragma unroll
-            for (int q = 0; q < 6; q++) s_v[q * n3p + pt] = hv[q];
-        }
         T tmp[5] = {0, 0, 0, 0, 0};
-#pragma unroll 1
-        for (int d = 0; d < 3; d++) {
-            T mme[3] = {0, 0, 0}, hm[3] = {0, 0, 0};
-            if (geo_lds) s_m = s_geo + 3 * d * n3p;
-            if (active) {
-                if (geo_lds) {
+        // the metric of direction d, from the registers that hold it since the load (geo_reg)
+        auto metric = [&](int d, int c) { return d == 0 ? gm[c] : (d == 1 ? gm[3 + c] : gm[6 + c]); };
+        // the node's viscous flux for metric m to s_f [4][n3p] (momentum, energy)
+        auto visc_flux = [&](const T* m, T* s_f) {
+            T f[5];
+            transformed_flux<T, false>(uc, pr, s, m, gas.hshift, f);
 #pragma unroll
-                    for (int c = 0; c < 3; c++) {
-                        hm[c] = s_m[c * n3p + pt];
-                        mme[c] = T(2) * hm[c];
+            for (int v = 1; v < 5; v++) s_f[(v - 1) * n3p + pt] = f[v];
+        };
+        auto visc_line = [&](int d, const T* s_f) {
+            const int idx = d == 0 ? i : (d == 1 ? j : k);
+            const auto ln = Lay<N>::line(d, i, j, k);
+#pragma unroll GALX_UNROLL_L
+            for (int l = 0; l <= N; l++) {
+                const T dh = M.dht(l, idx);
+                const int o = ln(l);
+#pragma unroll
+                for (int v = 1; v < 5; v++) ut[v] = ut[v] + dh * s_f[(v - 1) * n3p + o];
+            }
+        };
+        // the pairs of the node's line of direction d, metric halves hm of the node and s_m [3][n3p] of the line
+        auto pair_line = [&](int d, const T* hm, const T* s_m) {
+            const int idx = d == 0 ? i : (d == 1 ? j : k);
+            const auto ln = Lay<N>::line(d, i, j, k);
+            if (pair_lines && d < 2) {
+                // the two-point flux is symmetric, G(a,b) = G(b,a) bit for bit (sums and products of the
+                // same operands), so each pair of a line is formed once: the lane at line position a forms
+                // the pairs (a, a+s) for s = 1..(n-1)/2 (mod n) and reads the pair (a-s, a) from the lane s
+                // positions back with a cross-lane permute; for even n both ends of a pair (a, a+n/2) form
+                // it.  The diagonal, DVolSurf(a,a) = 0 up to rounding for Gauss-Lobatto (dg.f90:229-233),
+                // is left out.  About half the flux evaluations of the loop over all l below.
+                constexpr int msk = n - 1;                  // n is a power of two here
+                const int st = d == 0 ? 1 : n;              // lane distance between neighbours on the line
+                const int lane0 = (tid & 63) - idx * st;    // lane of line position 0
+                const T* dp = s_dp + idx;                   // s_dp[s*n + a] = DVolSurf((a+s) mod n, a)
+#pragma unroll
+                for (int s = 1; s <= n / 2; s++) {
+                    const int b = (idx + s) & msk;          // partner formed here
+                    const int o = ln(b);
+                    T Mo[3] = {s_m[o], s_m[n3p + o], s_m[2 * n3p + o]};
+                    T G[5];
+                    split_volume_flux_pi_half<T>(hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], s_v[o],
+                                                 s_v[n3p + o], s_v[2 * n3p + o], s_v[3 * n3p + o],
+                                                 s_v[4 * n3p + o], s_v[5 * n3p + o], hm, Mo, G);
+                    const T db = dp[s * n];
+                    if (2 * s < n) {
+                        const int src = lane0 + ((idx - s) & msk) * st;  // the lane that formed (a-s, a)
+                        const T da = dp[(n - s) * n];
+#pragma unroll
+                        for (int v = 0; v < 5; v++) {
+                            const T r = __shfl(G[v], src);
+                            tmp[v] = tmp[v] + db * G[v];
+                            tmp[v] = tmp[v] + da * r;
+                        }
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 5; v++) tmp[v] = tmp[v] + db * G[v];
                     }
-                } else {
+                }
+            } else {
+            // every partner l other than the node itself, l = idx + s (mod n) for s = 1..N: no per-lane
+            // branch.  VolInt_splitForm_Kernel (volint.f90:307-317) also adds the diagonal pair, whose
+            // DVolSurf(i,i) vanishes for Gauss-Lobatto up to rounding (dg.f90:229-233); the shared pairs above
+            // leave it out too (one flux of eight fewer on the k-lines at N=7: FP64 k_rhs 1.2 % faster)
+#pragma unroll GALX_UNROLL_SPLIT
+            for (int s = 1; s <= N; s++) {
+                const int l = idx + s <= N ? idx + s : idx + s - n;
+                const int o = ln(l);
+                T Mo[3] = {s_m[o], s_m[n3p + o], s_m[2 * n3p + o]};
+                T G[5];
+                split_volume_flux_pi_half<T>(hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], s_v[o], s_v[n3p + o],
+                                             s_v[2 * n3p + o], s_v[3 * n3p + o], s_v[4 * n3p + o],
+                                             s_v[5 * n3p + o], hm, Mo, G);
+                T dv = M.dvs(l, idx);
+#pragma unroll
+                for (int v = 0; v < 5; v++) tmp[v] = tmp[v] + dv * G[v];
+            }
+            }
+        };
+        if (visc_first) {
+#pragma unroll 1
+            for (int d = 0; d < 3; d++) {
+                // alternating buffers: the next direction's fluxes go to the one that no thread reads any more
+                T* s_f = s_w + (d & 1) * 4 * n3p;
+                if (active) {
+                    const T m[3] = {metric(d, 0), metric(d, 1), metric(d, 2)};
+                    visc_flux(m, s_f);
+                }
+                line_sync<N>(d);
+                if (active) visc_line(d, s_f);
+            }
+            __syncthreads();
+            // the sum of the pairs starts from half of the viscous terms (exact): no second set of accumulators
+            if (active) {
+#pragma unroll
+                for (int q = 0; q < 6; q++) s_v[q * n3p + pt] = hv[q];
+#pragma unroll
+                for (int v = 0; v < 5; v++) tmp[v] = T(0.5) * ut[v];
+            }
+#pragma unroll 1
+            for (int d = 0; d < 3; d++) {
+                T* s_m = s_w + 6 * n3p;
+                T hm[3] = {0, 0, 0};
+                if (active) {
 #pragma unroll
                     for (int c = 0; c < 3; c++) {
-                        // the prefetched values, kept in registers since the load (geo_reg)
-                        mme[c] = d == 0 ? gm[c] : (d == 1 ? gm[3 + c] : gm[6 + c]);
-                        hm[c] = T(0.5) * mme[c];
+                        hm[c] = T(0.5) * metric(d, c);
                         s_m[c * n3p + pt] = hm[c];
                     }
                 }
-                T f[5];
-                transformed_flux<T, false>(uc, pr, s, mme, gas.hshift, f);
-#pragma unroll
-                for (int v = 1; v < 5; v++) s_f[(v - 1) * n3p + pt] = f[v];
+                // s_v is read along the lines of d too: the k-lines' barrier here comes before any read across waves
+                line_sync<N>(d);
+                if (active) pair_line(d, hm, s_m);
+                line_sync<N>(d);
             }
-            // s_v (written after the lifting barrier) is read along the lines of d too: the k-lines' barrier below
-            // comes before any read across waves
-            line_sync<N>(d);
+#pragma unroll
+            for (int v = 0; v < 5; v++) ut[v] = T(2) * tmp[v];
+        } else {
             if (active) {
-                int idx = d == 0 ? i : (d == 1 ? j : k);
-                const auto ln = Lay<N>::line(d, i, j, k);
-#pragma unroll GALX_UNROLL_L
-                for (int l = 0; l <= N; l++) {
-                    T dh = M.dht(l, idx);
-                    const int o = ln(l);
 #pragma unroll
-                    for (int v = 1; v < 5; v++) ut[v] = ut[v] + dh * s_f[(v - 1) * n3p + o];
-                }
-                if (pair_lines && d < 2) {
-                    // the two-point flux is symmetric, G(a,b) = G(b,a) bit for bit (sums and products of the
-                    // same operands), so each pair of a line is formed once: the lane at line position a forms
-                    // the pairs (a, a+s) for s = 1..(n-1)/2 (mod n) and reads the pair (a-s, a) from the lane s
-                    // positions back with a cross-lane permute; for even n both ends of a pair (a, a+n/2) form
-                    // it.  The diagonal, DVolSurf(a,a) = 0 up to rounding for Gauss-Lobatto (dg.f90:229-233),
-                    // is left out.  About half the flux evaluations of the loop over all l below.
-                    constexpr int msk = n - 1;                  // n is a power of two here
-                    const int st = d == 0 ? 1 : n;              // lane distance between neighbours on the line
-                    const int lane0 = (tid & 63) - idx * st;    // lane of line position 0
-                    const T* dp = s_dp + idx;                   // s_dp[s*n + a] = DVolSurf((a+s) mod n, a)
+                for (int q = 0; q < 6; q++) s_v[q * n3p + pt] = hv[q];
+            }
+            T* s_f = s_w + (geo_lds ? 6 : 9) * n3p;
+#pragma unroll 1
+            for (int d = 0; d < 3; d++) {
+                T* s_m = geo_lds ? s_geo + 3 * d * n3p : s_w + 6 * n3p;
+                T m[3] = {0, 0, 0}, hm[3] = {0, 0, 0};
+                if (active) {
 #pragma unroll
-                    for (int s = 1; s <= n / 2; s++) {
-                        const int b = (idx + s) & msk;          // partner formed here
-                        const int o = ln(b);
-                        T Mo[3] = {s_m[o], s_m[n3p + o], s_m[2 * n3p + o]};
-                        T G[5];
-                        split_volume_flux_pi_half<T>(hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], s_v[o],
-                                                     s_v[n3p + o], s_v[2 * n3p + o], s_v[3 * n3p + o],
-                                                     s_v[4 * n3p + o], s_v[5 * n3p + o], hm, Mo, G);
-                        const T db = dp[s * n];
-                        if (2 * s < n) {
-                            const int src = lane0 + ((idx - s) & msk) * st;  // the lane that formed (a-s, a)
-                            const T da = dp[(n - s) * n];
-#pragma unroll
-                            for (int v = 0; v < 5; v++) {
-                                const T r = __shfl(G[v], src);
-                                tmp[v] = tmp[v] + db * G[v];
-                                tmp[v] = tmp[v] + da * r;
-                            }
+                    for (int c = 0; c < 3; c++) {
+                        if (geo_lds) {
+                            hm[c] = s_m[c * n3p + pt];
+                            m[c] = T(2) * hm[c];
                         } else {
-#pragma unroll
-                            for (int v = 0; v < 5; v++) tmp[v] = tmp[v] + db * G[v];
+                            m[c] = metric(d, c);
+                            hm[c] = T(0.5) * m[c];
+                            s_m[c * n3p + pt] = hm[c];
                         }
                     }
-                } else {
-                // every partner l other than the node itself, l = idx + s (mod n) for s = 1..N: no per-lane
-                // branch.  VolInt_splitForm_Kernel (volint.f90:307-317) also adds the diagonal pair, whose
-                // DVolSurf(i,i) vanishes for Gauss-Lobatto up to rounding (dg.f90:229-233); the shared pairs above
-                // leave it out too (one flux of eight fewer on the k-lines at N=7: FP64 k_rhs 1.2 % faster)
-#pragma unroll GALX_UNROLL_SPLIT
-                for (int s = 1; s <= N; s++) {
-                    const int l = idx + s <= N ? idx + s : idx + s - n;
-                    const int o = ln(l);
-                    T Mo[3] = {s_m[o], s_m[n3p + o], s_m[2 * n3p + o]};
-                    T G[5];
-                    split_volume_flux_pi_half<T>(hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], s_v[o], s_v[n3p + o],
-                                                 s_v[2 * n3p + o], s_v[3 * n3p + o], s_v[4 * n3p + o],
-                                                 s_v[5 * n3p + o], hm, Mo, G);
-                    T dv = M.dvs(l, idx);
-#pragma unroll
-                    for (int v = 0; v < 5; v++) tmp[v] = tmp[v] + dv * G[v];
+                    visc_flux(m, s_f);
                 }
+                line_sync<N>(d);
+                if (active) {
+                    visc_line(d, s_f);
+                    pair_line(d, hm, s_m);
                 }
+                line_sync<N>(d);
             }
-            line_sync<N>(d);
-        }
 #pragma unroll
-        for (int v = 0; v < 5; v++) ut[v] = ut[v] + T(2) * tmp[v];
+            for (int v = 0; v < 5; v++) ut[v] = ut[v] + T(2) * tmp[v];
+        }
         // enthalpy offset (mixed form): the pair fluxes carried H - href, and the energy flux q {H} is
         // q {H - href} + href q, so the energy sum takes href times the mass sum back once per node.  The FP32
         // products then hold the enthalpy fluctuation at full precision instead of rounding q {H}, whose mean part
@@ -1150,7 +1283,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T>::value)
         long side = c >> 3;
         int flip = c & 7;
         int pq = mesh.inv[(flip * 6 + ls - 1) * n2 + ab];
-        T Uo[5], fvo[4], Un[5], fvn[4];
+        T Uo[5], Un[5], fv[8];
         {
             // the record the neighbour reads.  Mixed form: from the own slot of the FP32 trace buffer (0.5 % faster
             // at N=7 on MI355X, though it reads 15 B/DOF more from HBM than the gather of the FP64 state, which
@@ -1173,18 +1306,22 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T>::value)
             }
         }
         const TT* vo = vtr + ((side * 2 + (flip ? 1 : 0)) * 4) * n2 + pq;  // written by k_lift of this element
+        if (!lean) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) fvo[q] = T(vo[q * n2]);
+            for (int q = 0; q < 4; q++) fv[q] = T(vo[q * n2]);
+        }
         const long nslot = side * 2 + (flip ? 0 : 1);
         const T* un = s_nb + (ls - 1) * 5 * n2 + ab;
         const TT* vn = vtr + nslot * 4 * n2 + pq;
 #pragma unroll
         for (int v = 0; v < 5; v++) Un[v] = un[v * n2];
+        if (!lean) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) fvn[q] = T(vn[q * n2]);
+            for (int q = 0; q < 4; q++) fv[4 + q] = T(vn[q * n2]);
+        }
         T F[5];
-        face_flux<N, T, TT, SPLIT, RIEMANN>(Uo, fvo, Un, fvn, GeoOf<T>::fgeo(mesh) + side * 10 * n2 + pq, n2, flip,
-                                            gas, F);
+        face_flux<N, T, TT, SPLIT, RIEMANN, lean>(Uo, Un, fv, vo, vn, GeoOf<T>::fgeo(mesh) + side * 10 * n2 + pq, n2,
+                                                  flip, gas, F);
         T sg = flip ? T(-1) : T(1);
 #pragma unroll
         for (int v = 0; v < 5; v++) s_res[(ls - 1) * 5 * n2 + v * n2 + ab] = sg * F[v];

@@ -370,7 +370,7 @@ __device__ __forceinline__ void plane_face_flux(int e, const FaceTask& f, int no
 {
     constexpr int n2 = Pl<N>::n2, n3 = Pl<N>::n3;
     const long own = f.side * 2 + (f.flip ? 1 : 0), nb = f.side * 2 + (f.flip ? 0 : 1);
-    T Uo[5], Un[5], fvo[4], fvn[4];
+    T Uo[5], Un[5], fv[8];
     {
         const double* uo = U + (long)e * 5 * n3 + node;
         double c[5], tr[5];
@@ -382,13 +382,8 @@ __device__ __forceinline__ void plane_face_flux(int e, const FaceTask& f, int no
     }
 #pragma unroll
     for (int v = 0; v < 5; v++) Un[v] = T(utr[(nb * 5 + v) * n2 + f.pq]);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        fvo[q] = T(vtr[(own * 4 + q) * n2 + f.pq]);
-        fvn[q] = T(vtr[(nb * 4 + q) * n2 + f.pq]);
-    }
-    face_flux<N, T, TT, SPLIT, RIEMANN>(Uo, fvo, Un, fvn, GeoOf<T>::fgeo(mesh) + f.side * 10 * n2 + f.pq, n2, f.flip,
-                                        gas, F);
+    face_flux<N, T, TT, SPLIT, RIEMANN, true>(Uo, Un, fv, vtr + own * 4 * n2 + f.pq, vtr + nb * 4 * n2 + f.pq,
+                                              GeoOf<T>::fgeo(mesh) + f.side * 10 * n2 + f.pq, n2, f.flip, gas, F);
     const T sg = f.flip ? T(-1) : T(1);
 #pragma unroll
     for (int v = 0; v < 5; v++) F[v] = sg * F[v];
