@@ -204,16 +204,19 @@ __global__ void __launch_bounds__(256) k_source(long nDOF, int n3, const double*
 #pragma unroll
     for (int v = 0; v < 5; v++) {
         double S = sc.c[v][0] * cs + sc.c[v][1] * sn2 + sc.c[v][2] * sn;
-        double o = p[v * n3];
+        const double o = mode == 0 || mRKA != 0.0 ? p[v * n3] : 0.0;
         p[v * n3] = mode == 0 ? o + S : o * mRKA + S;
     }
 }
 
-// per-block sums of the pressure over all nodes (element planes), for the pressure offset of the mixed form; the
-// host adds the block sums in order, so the offset, and with it the mixed-form trajectory, is the same every run
-// per-block sums of the pressure and of the enthalpy H = (E+p)/rho (the mixed form's offsets): out[2b], out[2b+1]
-__global__ void __launch_bounds__(256) k_pressure_sum(long nDOF, int n3, double kappa, const double* __restrict__ U,
-                                                      double* __restrict__ out)
+// k_ref_to_planes with the per-block sums of the pressure and of the enthalpy H = (E+p)/rho over the nodes (the mixed
+// form's offsets) to out[2b], out[2b+1], host memory that the device writes; the host adds the block sums in order, so the
+// offsets, and with them the mixed-form trajectory, are the same every run.  (A tree of the block sums on the device moves
+// the offsets by one unit in the last place, which the FP32 roundings behind them spread to 5e-10 of the state in a few
+// steps.)
+__global__ void __launch_bounds__(256) k_ref_to_planes_sum(long nDOF, int n3, double kappa,
+                                                           const double* __restrict__ src, double* __restrict__ dst,
+                                                           double* __restrict__ out)
 {
     __shared__ double s[2][4];
     long x = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -221,11 +224,14 @@ __global__ void __launch_bounds__(256) k_pressure_sum(long nDOF, int n3, double 
     if (x < nDOF) {
         long e = x / n3;
         int node = (int)(x - e * n3);
-        const double* u = U + e * 5 * n3 + node;
-        double rho = u[0], sRho = 1.0 / rho;
-        double m1 = u[n3], m2 = u[2 * n3], m3 = u[3 * n3];
-        p = (kappa - 1.0) * (u[4 * n3] - 0.5 * (m1 * m1 + m2 * m2 + m3 * m3) * sRho);
-        h = (u[4 * n3] + p) * sRho;
+        double c[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++) c[v] = src[5 * x + v];
+#pragma unroll
+        for (int v = 0; v < 5; v++) dst[(e * 5 + v) * n3 + node] = c[v];
+        double sRho = 1.0 / c[0];
+        p = (kappa - 1.0) * (c[4] - 0.5 * (c[1] * c[1] + c[2] * c[2] + c[3] * c[3]) * sRho);
+        h = (c[4] + p) * sRho;
     }
     for (int off = 32; off > 0; off >>= 1) {
         p += __shfl_xor(p, off, 64);
@@ -250,6 +256,7 @@ struct KernelSet {
     int block = 0;
     size_t (*ws_bytes)(int) = nullptr;  // workspace of a mesh of that many elements (the plane kernels)
     void (*trace)(hipStream_t, int, const double*, Mesh, void*, GasD) = nullptr;
+    void (*set_state)(hipStream_t, int, const double*, double*, Mesh, double*, GasD) = nullptr;  // FP64 form only
     void (*lift)(hipStream_t, int, const double*, Mesh, const void*, void*, const void*, GasD, double, double) = nullptr;
     void (*rhs)(hipStream_t, int, const double*, double*, Mesh, const void*, const void*, void*, double*, double*,
                 const void*, GasD, int, double, double, Stage) = nullptr;
@@ -271,6 +278,10 @@ struct Launch {
     static void trace(hipStream_t s, int nE, const double* U, Mesh m, void* utr, GasD g)
     {
         hipLaunchKernelGGL((k_trace<N, T>), dim3(nE), dim3(D::block), 0, s, U, m, (T*)utr, g);
+    }
+    static void set_state(hipStream_t s, int nE, const double* src, double* U, Mesh m, double* utr, GasD g)
+    {
+        hipLaunchKernelGGL((k_set_state<N>), dim3(nE), dim3(D::block), 0, s, src, U, m, utr, g);
     }
     static void lift(hipStream_t s, int nE, const double* U, Mesh m, const void* utr, void* vtr, const void* mats,
                      GasD g, double LHm, double LHp)
@@ -344,6 +355,7 @@ struct Launch {
         k.block = D::block;
         k.ws_bytes = &ws_bytes;
         k.trace = &trace;
+        if constexpr (sizeof(T) == 8) k.set_state = &set_state;
         k.lift = &lift;
         k.rhs = &rhs;
         k.dt = &dt;
@@ -462,8 +474,10 @@ struct galx_ctx {
     void* dWs = nullptr;  // per-element workspace of the plane kernels
     int *dConn = nullptr, *dInv = nullptr;
     void *dUtr[2] = {nullptr, nullptr}, *dVtr = nullptr, *dMats = nullptr;
-    double *dDtc = nullptr, *dDtv = nullptr, *dDtOut = nullptr;
+    double *dDtc = nullptr, *dDtv = nullptr;
     int* dErr = nullptr;
+    double* hOut = nullptr;  // pinned host memory for the few doubles that a kernel hands to the host
+    bool kZero = false;      // the LSERK register holds zero, whatever its memory holds
     int cur = 0;
     bool meshSet = false, stateSet = false, utValid = false;
     // discrete adjoint: cotangents, face traces and the recorded forward trajectory (element planes)
@@ -487,7 +501,7 @@ struct galx_ctx {
     int srcFunc = 0;
     SourceCoefs src{};
     double* dSrcX = nullptr;
-    double* dPsum = nullptr;  // per-block pressure sums (mixed form's offset)
+    double* hPsum = nullptr;  // pinned: per-block pressure and enthalpy sums (mixed form's offsets)
     long long bytes = 0;
     bool timing = false;
     std::map<std::string, Timer> timers;
@@ -615,7 +629,7 @@ struct Staging {
 static void free_mesh(galx_ctx* c)
 {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    double** pd[] = {&c->dU, &c->dK, &c->dGeo, &c->dFgeo, &c->dSgeo, &c->dDtc, &c->dDtv, &c->dDtOut};
+    double** pd[] = {&c->dU, &c->dK, &c->dGeo, &c->dFgeo, &c->dSgeo, &c->dDtc, &c->dDtv};
     for (double** p : pd) {
         dfree(*p);
         *p = nullptr;
@@ -661,7 +675,6 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
     if ((rc = dalloc(c, (char**)&c->dVtr, 2 * 4 * nfn * c->tsz))) return rc;
     if ((rc = dalloc(c, &c->dDtc, nElems * sizeof(double)))) return rc;
     if ((rc = dalloc(c, &c->dDtv, nElems * sizeof(double)))) return rc;
-    if ((rc = dalloc(c, &c->dDtOut, 4 * sizeof(double)))) return rc;
     if ((rc = dalloc(c, &c->dErr, sizeof(int)))) return rc;
     if (const size_t b = c->ks.ws_bytes(nElems); b && (rc = dalloc(c, (char**)&c->dWs, b))) return rc;
     if (c->tsz == 4) {
@@ -669,12 +682,13 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
         if ((rc = dalloc(c, &c->dFgeo32, 10 * nfn * sizeof(float)))) return rc;
         if ((rc = dalloc(c, &c->dSgeo32, 10L * nElems * ns * sizeof(float)))) return rc;
     }
+    HIPCHK(hipMemset(c->dErr, 0, sizeof(int)));
     HIPCHK(hipMemcpy(c->dConn, conn.data(), conn.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->dInv, inv.data(), inv.size() * sizeof(int), hipMemcpyHostToDevice));
     // geometry into element / side planes, in chunks through two pinned staging buffers: the host fills one while
     // the copy of the other runs.  The surface-node copy of the element geometry (k_lift's metrics) comes from the
     // same planes.
-    const long chunkE = 1024, chunkS = 4096;  // 66 MB per staging buffer at N=7
+    const long chunkE = std::min(1024, nElems), chunkS = std::min(4096, nSides);  // at most 66 MB a buffer at N=7
     const size_t stageB = std::max(10 * chunkE * (n3 + ns), 10 * chunkS * n2) * sizeof(double);
     Staging stg;
     if ((rc = stg.init(stageB))) return rc;
@@ -824,6 +838,11 @@ int galx_create(const galx_config* cfg, galx_ctx** out)
         galx_destroy(c);
         return fail(GALX_E_HIP, "hipMemcpy: %s", hipGetErrorString(e));
     }
+    if (hipHostMalloc((void**)&c->hOut, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        c->hOut = nullptr;
+        galx_destroy(c);
+        return fail(GALX_E_NOMEM, "hipHostMalloc failed");
+    }
     *out = c;
     return GALX_OK;
 }
@@ -835,16 +854,18 @@ int galx_destroy(galx_ctx* c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     flush_timers(c);
     void* ps[] = {c->dU,      c->dK,    c->dUt,   c->dScratch, c->dGeo,  c->dFgeo, c->dSgeo, c->dConn, c->dInv,
-                  c->dUtr[0], c->dUtr[1], c->dVtr, c->dMats,    c->dDtc, c->dDtv,  c->dDtOut, c->dErr,
+                  c->dUtr[0], c->dUtr[1], c->dVtr, c->dMats,    c->dDtc, c->dDtv,  c->dErr,
                   c->dGeo32,  c->dFgeo32, c->dSgeo32, c->dWs};
     for (void* p : ps) dfree(p);
     void* pa[] = {c->dKbar,    c->dUbar,   c->dMutr,    c->dNghtr, c->dUfinal,
-                  c->dGrad,    c->dGradRef, c->dMats64, c->dTr64,  c->dSrcX, c->dPsum};
+                  c->dGrad,    c->dGradRef, c->dMats64, c->dTr64,  c->dSrcX};
     for (void* p : pa) dfree(p);
     for (double* p : c->ckpt) dfree(p);
     for (double* p : c->stages) dfree(p);
     for (double* p : c->stageTr) dfree(p);
     for (double* p : c->steps) dfree(p);
+    if (c->hOut) (void)hipHostFree(c->hOut);
+    if (c->hPsum) (void)hipHostFree(c->hPsum);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return GALX_OK;
@@ -910,34 +931,37 @@ int galx_set_mesh(galx_ctx* c, int nElems, int nSides, const int* E2S, const int
 }
 
 
-static int after_state(galx_ctx* c)
+// the context state from dSrc in the reference layout (device memory), with its traces; the LSERK register starts at zero
+static int state_in(galx_ctx* c, const double* dSrc)
 {
     c->trajValid = false;  // a recorded trajectory no longer ends at the context state
-    HIPCHK(hipMemsetAsync(c->dK, 0, 5L * c->nElems * c->n3 * sizeof(double), c->stream));
+    c->kZero = true;
     c->cur = 0;
     c->pref = 0.0;
     c->href = 0.0;
-    if (c->cfg.precision == GALX_PREC_MIXED) {
+    if (c->cfg.precision == GALX_PREC_FP64) {
+        TimerScope ts(c, "trace");
+        c->ks.set_state(c->stream, c->nElems, dSrc, c->dU, mesh_of(c), (double*)c->dUtr[0], gas_of(c));
+    } else {
         long nDOF = (long)c->nElems * c->n3;
         const long nb = (nDOF + 255) / 256;
-        int rc;
-        if ((rc = dalloc(c, &c->dPsum, 2 * nb * sizeof(double)))) return rc;
-        k_pressure_sum<<<dim3((unsigned)nb), dim3(256), 0, c->stream>>>(nDOF, c->n3, c->cfg.kappa, c->dU, c->dPsum);
+        if (!c->hPsum && hipHostMalloc((void**)&c->hPsum, 2 * nb * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+            c->hPsum = nullptr;
+            return fail(GALX_E_NOMEM, "hipHostMalloc(%ld) failed", 2 * nb * (long)sizeof(double));
+        }
+        k_ref_to_planes_sum<<<dim3((unsigned)nb), dim3(256), 0, c->stream>>>(nDOF, c->n3, c->cfg.kappa, dSrc, c->dU,
+                                                                             c->hPsum);
         HIPCHK(hipGetLastError());
-        std::vector<double> part(2 * nb);
-        HIPCHK(hipMemcpyAsync(part.data(), c->dPsum, 2 * nb * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
         double sp = 0.0, sh = 0.0;
         for (long b = 0; b < nb; b++) {
-            sp += part[2 * b];
-            sh += part[2 * b + 1];
+            sp += c->hPsum[2 * b];
+            sh += c->hPsum[2 * b + 1];
         }
         c->pref = sp / (double)nDOF;
         c->href = sh / (double)nDOF;
         if (!(c->pref == c->pref)) c->pref = 0.0;
         if (!(c->href == c->href)) c->href = 0.0;
-    }
-    {
         TimerScope ts(c, "trace");
         c->ks.trace(c->stream, c->nElems, c->dU, mesh_of(c), c->dUtr[0], gas_of(c));
     }
@@ -953,10 +977,7 @@ int galx_set_state_device(galx_ctx* c, const double* dU)
     if (!c || !dU) return fail(GALX_E_ARG, "null argument");
     if (!c->meshSet) return fail(GALX_E_STATE, "set_mesh first");
     HIPCHK(hipSetDevice(c->cfg.device));
-    long nDOF = (long)c->nElems * c->n3;
-    k_ref_to_planes<<<dim3((unsigned)((nDOF + 255) / 256)), dim3(256), 0, c->stream>>>(nDOF, c->n3, dU, c->dU);
-    HIPCHK(hipGetLastError());
-    return after_state(c);
+    return state_in(c, dU);
 }
 
 // CalcSource's terms (src/equations/navierstokes/idealgas/exactfunc.f90:946-1111) as one coefficient table per
@@ -1033,9 +1054,7 @@ int galx_set_state(galx_ctx* c, const double* U)
     int rc;
     if ((rc = dalloc(c, &c->dScratch, 5 * nDOF * sizeof(double)))) return rc;
     HIPCHK(hipMemcpyAsync(c->dScratch, U, 5 * nDOF * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    k_ref_to_planes<<<dim3((unsigned)((nDOF + 255) / 256)), dim3(256), 0, c->stream>>>(nDOF, c->n3, c->dScratch, c->dU);
-    HIPCHK(hipGetLastError());
-    return after_state(c);
+    return state_in(c, c->dScratch);
 }
 
 int galx_get_state_device(galx_ctx* c, double* dU)
@@ -1092,6 +1111,10 @@ static void launch_source(galx_ctx* c, double t, int mode, double mRKA)
 static void launch_rhs(galx_ctx* c, Stage st, double t, const double* U = nullptr, double* Uout = nullptr,
                        const void* utr = nullptr, void* utr_next = nullptr)
 {
+    if (st.mode == 1) {
+        if (c->kZero) st.mRKA = 0.0;  // the kernels then leave the register's memory unread
+        c->kZero = false;
+    }
     if (c->srcFunc && st.mode == 1) {
         launch_source(c, t, 1, st.mRKA);
         st.mRKA = 1.0;
@@ -1286,19 +1309,16 @@ int galx_calc_dt(galx_ctx* c, double* dt, int* errType)
     double DFL = c->cfg.DFLScale * DFL_ALPHA_GL[Nd - 1] * 1.853 / ((2.0 * N + 1.0) * (2.0 * N + 1.0));
     double kp = c->cfg.kappa / c->cfg.Pr;
     double KPmax = kp > 4.0 / 3.0 ? kp : 4.0 / 3.0;
-    HIPCHK(hipMemsetAsync(c->dErr, 0, sizeof(int), c->stream));
     {
         TimerScope ts(c, "dt");
         c->ks.dt(c->stream, c->nElems, c->dU, c->dGeo, c->cfg.kappa, c->cfg.mu0, KPmax, CFL, DFL, c->dDtc, c->dDtv,
                  c->dErr);
-        k_dt_reduce<<<dim3(1), dim3(1024), 0, c->stream>>>(c->nElems, c->dDtc, c->dDtv, c->dErr, c->dDtOut);
+        k_dt_reduce<<<dim3(1), dim3(1024), 0, c->stream>>>(c->nElems, c->dDtc, c->dDtv, c->dErr, c->hOut);
     }
     HIPCHK(hipGetLastError());
-    double out[4];
-    HIPCHK(hipMemcpyAsync(out, c->dDtOut, sizeof(out), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    *dt = out[2];
-    *errType = (int)out[3];
+    *dt = c->hOut[0];
+    *errType = (int)c->hOut[1];
     return GALX_OK;
 }
 
@@ -1606,7 +1626,7 @@ static int adj_finish(galx_ctx* c, const double* pending)
     HIPCHK(hipMemcpyAsync(c->dU, c->dUfinal, ub, hipMemcpyDeviceToDevice, c->stream));
     c->cur = 0;
     c->ks.trace(c->stream, c->nElems, c->dU, m, c->dUtr[0], gd);
-    HIPCHK(hipMemsetAsync(c->dK, 0, ub, c->stream));
+    c->kZero = true;
     HIPCHK(hipGetLastError());
     c->utValid = false;
     return GALX_OK;

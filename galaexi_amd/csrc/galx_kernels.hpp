@@ -187,7 +187,8 @@ struct GeoOf<float> {
 
 struct Stage {
     double mRKA, bdt;
-    int mode;  // 0: write Ut; 1: LSERK register update
+    int mode;  // 0: write Ut; 1: LSERK register update, K = mRKA*K + Ut; with mRKA = 0 (the first stage of a step, or a
+               // register that is zero) K is not read: 40 of the stage's 500 bytes per node
 };
 
 // matrices staged in LDS: D_T (transpose of D), D_Hat_T, DVolSurf, all (0:N,0:N); dt(a,b), dht(a,b), dvs(a,b)
@@ -706,6 +707,41 @@ __global__ void __launch_bounds__(Dm<N>::block)
 #pragma unroll
         for (int v = 0; v < 5; v++) cv[v] = u[v * n3];
         store_trace(o, n2, cv, gd);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// k_set_state: a state in the reference layout U(5,n3,nElems) to the element planes and its U traces (FP64; the mixed
+// form's traces need the mean pressure of the whole state first).  Bound by its bytes, 110 per node at N = 7: 5.2 TB/s
+// on 32^3 elements.  One pass instead of a transposition, a clear of the LSERK register and a trace pass that read the
+// state again: galx_set_state_device 576 -> 369 us there, 19 -> 14 us on 8^3 elements at N = 3.
+// ---------------------------------------------------------------------------------------------------------
+template <int N>
+__global__ void __launch_bounds__(Dm<N>::block)
+    k_set_state(const double* __restrict__ src, double* __restrict__ U, Mesh mesh, double* __restrict__ utr, GasD gd)
+{
+    using D = Dm<N>;
+    constexpr int n = D::n, n2 = D::n2, n3 = D::n3;
+    const int e = blockIdx.x;
+    for (int node = threadIdx.x; node < n3; node += D::block) {
+        const double* s = src + ((long)e * n3 + node) * 5;
+        double* u = U + (long)e * 5 * n3 + node;
+        double c[5], tr[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++) c[v] = s[v];
+#pragma unroll
+        for (int v = 0; v < 5; v++) u[v * n3] = c[v];
+        trace_record<false>(c, gd.kappa, gd.pref, tr);
+        const int i = node % n, j = (node / n) % n, k = node / n2;
+#pragma unroll
+        for (int ls = 1; ls <= 6; ls++) {
+            int ab;
+            if (!on_face<N>(ls, i, j, k, ab)) continue;
+            const int cn = mesh.conn[e * 6 + ls - 1], flip = cn & 7;
+            double* o = utr + (2L * (cn >> 3) + (flip ? 1 : 0)) * 5 * n2 + mesh.inv[(flip * 6 + ls - 1) * n2 + ab];
+#pragma unroll
+            for (int v = 0; v < 5; v++) o[v * n2] = tr[v];
+        }
     }
 }
 
@@ -1344,11 +1380,12 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
         const double sJd = geo_reg ? double(gm[9]) : ge[9 * n3];
         if (st.mode != 0) {
             const double* uo = U + (long)e * 5 * n3 + tid;
+            if (st.mRKA != 0.0) {
 #pragma unroll
-            for (int v = 0; v < 5; v++) {
-                kv[v] = ut_out[v * n3];
-                uv[v] = uo[v * n3];
+                for (int v = 0; v < 5; v++) kv[v] = ut_out[v * n3];
             }
+#pragma unroll
+            for (int v = 0; v < 5; v++) uv[v] = uo[v * n3];
         }
 #pragma unroll
         for (int v = 0; v < 5; v++) {
@@ -1399,7 +1436,7 @@ template <int N>
 __global__ void __launch_bounds__(Dm<N>::block)
     k_dt_elem(const double* __restrict__ U, const double* __restrict__ geo, double kappa, double mu0, double KPmax,
               double CFLScale, double DFLScale, double* __restrict__ dtc, double* __restrict__ dtv,
-              int* __restrict__ err)
+              int* __restrict__ err)  // |= 1 on a non-positive density; zero on entry (k_dt_reduce leaves it so)
 {
     using D = Dm<N>;
     constexpr int n3 = D::n3;
@@ -1454,9 +1491,10 @@ __global__ void __launch_bounds__(Dm<N>::block)
     }
 }
 
+// the minima over the elements and errType to `out`, in host memory that the device writes (one copy and its launch fewer:
+// the call waits for the stream anyway); err is left at zero for the next call
 __global__ void __launch_bounds__(1024) k_dt_reduce(int nElems, const double* __restrict__ dtc,
-                                                    const double* __restrict__ dtv, int* __restrict__ err,
-                                                    double* __restrict__ out)
+                                                    const double* __restrict__ dtv, int* __restrict__ err, double* out)
 {
     __shared__ double s[2][16];
     __shared__ int s_nan[2];
@@ -1465,6 +1503,7 @@ __global__ void __launch_bounds__(1024) k_dt_reduce(int nElems, const double* __
     __syncthreads();
     double a = 1e300, b = 1e300;
     int na = 0, nb = 0;
+#pragma unroll 4
     for (int x = tid; x < nElems; x += 1024) {
         double va = dtc[x], vb = dtv[x];
         if (va != va) na = 1; else a = fmin(a, va);
@@ -1486,11 +1525,9 @@ __global__ void __launch_bounds__(1024) k_dt_reduce(int nElems, const double* __
             a = fmin(a, s[0][w]);
             b = fmin(b, s[1][w]);
         }
-        out[0] = a;
-        out[1] = b;
-        out[2] = a < b ? a : b;
-        int ev = err[0] ? 1 : (s_nan[0] ? 2 : (s_nan[1] ? 3 : 0));
-        out[3] = double(ev);
+        out[0] = a < b ? a : b;
+        out[1] = double(err[0] ? 1 : (s_nan[0] ? 2 : (s_nan[1] ? 3 : 0)));
+        err[0] = 0;
     }
 }
 
