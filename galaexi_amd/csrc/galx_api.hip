@@ -273,6 +273,7 @@ struct Launch {
     using D = Dm<N>;
     // has the degree kernels with one element per workgroup, and plane kernels
     static constexpr bool whole = N < GALX_PLANE_DEGREE, planes = use_planes<N, T>(1);
+    static dim3 pack_grid(int nE) { return dim3((nE + Pack<N>::of(nE) - 1) / Pack<N>::of(nE)); }
     static dim3 plane_grid(int nE) { return dim3(8 * plane_per_xcd(nE * Pl<N>::groups)); }
     static size_t ws_bytes(int nE) { return use_planes<N, T>(nE) ? (size_t)nE * Pl<N>::ws * sizeof(T) : 0; }
     static void trace(hipStream_t s, int nE, const double* U, Mesh m, void* utr, GasD g)
@@ -293,8 +294,8 @@ struct Launch {
                 return;
             }
         if constexpr (whole)
-            hipLaunchKernelGGL((k_lift<N, T, T>), dim3(nE), dim3(D::block), 0, s, U, m, (const T*)utr, (T*)vtr,
-                               (const T*)mats, g, T(LHm), T(LHp));
+            hipLaunchKernelGGL((k_lift<N, T, T>), pack_grid(nE), dim3(D::block), 0, s, Pack<N>::of(nE),
+                               nE, U, m, (const T*)utr, (T*)vtr, (const T*)mats, g, T(LHm), T(LHp));
     }
     template <int RIE>
     static void rhs_r(hipStream_t s, int nE, const double* U, double* Uout, Mesh m, const void* utr, const void* vtr,
@@ -309,9 +310,9 @@ struct Launch {
                 return;
             }
         if constexpr (whole)
-            hipLaunchKernelGGL((k_rhs<N, T, T, SPLIT, RIE>), dim3(nE), dim3(D::block), 0, s, U, Uout, m,
-                               (const T*)utr, (const T*)vtr, (T*)utr_next, Ut, K, (const T*)mats, g, T(LHm), T(LHp),
-                               st);
+            hipLaunchKernelGGL((k_rhs<N, T, T, SPLIT, RIE>), pack_grid(nE), dim3(D::block), 0, s,
+                               Pack<N>::of(nE), nE, U, Uout, m, (const T*)utr, (const T*)vtr, (T*)utr_next, Ut, K,
+                               (const T*)mats, g, T(LHm), T(LHp), st);
     }
     static void rhs(hipStream_t s, int nE, const double* U, double* Uout, Mesh m, const void* utr, const void* vtr,
                     void* utr_next, double* Ut, double* K, const void* mats, GasD g, int riemann, double LHm,

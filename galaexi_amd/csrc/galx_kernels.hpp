@@ -44,6 +44,43 @@ struct Dm {
     static constexpr int ft = (nf + block - 1) / block;
 };
 
+// Elements per workgroup of k_lift and k_rhs (their epb).  An element of N = 1 or 2 fills 8 or 27 lanes of the one wave
+// it works in, so these degrees put `most` of them into a workgroup: half as many waves at N = 2 and a quarter at N = 1
+// (8 per wave there measured the same as 4, with twice the passes over their face nodes; 2 per wave 24 % slower than 4).
+// us of k_lift + k_rhs with one element per wave and packed: N = 1 split LF 1401 -> 664 at 64^3 elements, 164 -> 81 at
+// 32^3, 26.9 -> 23.6 at 13^3, 20.8 -> 20.7 at 10^3, 17.3 -> 20.6 at 6^3; N = 2 weak LF 226 -> 212 at 32^3, 36.8 -> 35.3
+// at 16^3, 30.0 -> 30.2 at 13^3, 21.9 -> 24.1 at 10^3 and split Roe 247 -> 215 at 32^3, 32.9 -> 32.6 at 13^3.  Under
+// the line one element per wave leaves less than two waves per SIMD, and its face nodes in one pass are the shorter
+// chain.
+template <int N>
+struct Pack {
+    static constexpr int most = N == 1 ? 4 : (N == 2 ? 2 : 1);
+    static constexpr int line = 2048;  // elements of the mesh from which the workgroups are packed
+    static_assert(most * Dm<N>::n3 <= Dm<N>::block, "one volume node per thread");
+    static int of(int nElems) { return nElems >= line ? most : 1; }
+
+    int le, e, node;  // the element of the thread's node in the workgroup and in the mesh, the node in it
+    bool active;
+    __device__ __forceinline__ Pack(int tid, int epb, int nElems)
+    {
+        constexpr int n3 = Dm<N>::n3;
+        le = most == 1 ? 0 : min(tid / n3, most - 1);
+        node = tid - le * n3;
+        e = most == 1 ? (int)blockIdx.x : (int)blockIdx.x * epb + le;
+        active = node < n3 && (most == 1 || (le < epb && e < nElems));
+    }
+    // face nodes of the workgroup: x = le * nf + t is face node t of element elem(le)
+    __device__ static __forceinline__ int faces(int epb, int nElems)
+    {
+        return most == 1 ? Dm<N>::nf : Dm<N>::nf * min(epb, nElems - (int)blockIdx.x * epb);
+    }
+    __device__ static __forceinline__ int face_le(int x) { return most == 1 ? 0 : x / Dm<N>::nf; }
+    __device__ static __forceinline__ int elem(int le, int epb)
+    {
+        return most == 1 ? (int)blockIdx.x : (int)blockIdx.x * epb + le;
+    }
+};
+
 // nodes on the element surface, n^3 - (n-2)^3 of them
 __host__ __device__ constexpr int surface_count(int N) { return 2 * (N + 1) * (N + 1) + (N - 1) * 4 * N; }
 
@@ -328,6 +365,22 @@ __device__ __forceinline__ void lift_face_fluxes(int e, int tid, const Mesh& mes
         LiftOperands<T> p;
         load_lift_operands<N, T, TT>(f, mesh, utr, p);
         lift_face_task<N, T>(f, p, s_lift, s_lflux, gas, s_nb);
+    }
+}
+
+// the same for the elements of a packed workgroup, whose LDS slices lie `slice` (s_lift, s_lflux) and nb_slice apart
+template <int N, typename T, typename TT>
+__device__ __forceinline__ void lift_face_fluxes_packed(int tid, int epb, int nElems, const Mesh& mesh,
+                                                        const TT* __restrict__ utr, const T* s_lift, T* s_lflux,
+                                                        int slice, const Gas<T>& gas, T* s_nb, int nb_slice)
+{
+    const int nx = Pack<N>::faces(epb, nElems);
+    for (int x = tid; x < nx; x += Dm<N>::block) {
+        const int le = Pack<N>::face_le(x);
+        const FaceTask f = face_task<N>(Pack<N>::elem(le, epb), x - le * Dm<N>::nf, mesh);
+        LiftOperands<T> p;
+        load_lift_operands<N, T, TT>(f, mesh, utr, p);
+        lift_face_task<N, T>(f, p, s_lift + le * slice, s_lflux + le * slice, gas, s_nb ? s_nb + le * nb_slice : nullptr);
     }
 }
 
@@ -771,7 +824,7 @@ struct LiftWaves {
 
 template <int N, typename T, typename TT>
 __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
-    k_lift(const double* __restrict__ U, Mesh mesh, const TT* __restrict__ utr, TT* __restrict__ vtr,
+    k_lift(int epb, int nElems, const double* __restrict__ U, Mesh mesh, const TT* __restrict__ utr, TT* __restrict__ vtr,
            const T* __restrict__ mats, GasD gd, T LHm, T LHp)
 {
     using D = Dm<N>;
@@ -780,11 +833,14 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     constexpr int n3p = Lay<N>::n3;
     // own (u,v,w,T) | lifting fluxes, then the own face nodes' stress and heat flux (9 values, not the 12 gradients)
     constexpr int w_f = 6 * 9 * n2 > 6 * 7 * n2 ? 6 * 9 * n2 : 6 * 7 * n2;
-    __shared__ T s_buf[4 * n3p + w_f];
+    constexpr int slice = 4 * n3p + w_f;
+    __shared__ T s_buf[Pack<N>::most * slice];
     __shared__ MatsD<N, T> M;
-    const int e = blockIdx.x, tid = threadIdx.x;
-    T* s_lift = s_buf;
-    T* s_lflux = s_buf + 4 * n3p;
+    const int tid = threadIdx.x;
+    const Pack<N> own(tid, epb, nElems);
+    const int e = own.e;
+    T* s_lift = s_buf + own.le * slice;
+    T* s_lflux = s_lift + 4 * n3p;
     load_mats<N, T>(M, mats, tid, D::block);
     const Gas<T> gas = make_gas<T>(gd);
     T uc[5], pr[6], H;
@@ -793,13 +849,13 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     // interior nodes' gradients and metrics are skipped (measured on MI355X at N=7 against every node's gradient:
     // 8 % faster in FP64, 12 % in the mixed form; with the metrics from the volume planes, whose 64-byte rows all
     // hold surface nodes, 1.8 % faster in FP64 and 3 % slower in the mixed form)
-    const bool gnode = tid < Surf<N>::count;
-    const int gn = gnode ? surface_node<N>(tid) : 0;
+    const bool gnode = own.active && own.node < Surf<N>::count;
+    const int gn = gnode ? surface_node<N>(own.node) : 0;
     T gm[10];
-    if (gnode) load_surf_geo<N, T>(e, tid, mesh, gm);
-    if (tid < n3) {
-        load_state<N, T>(e, tid, U, gd, uc, pr, H);
-        const int pt = Lay<N>::at(tid);
+    if (gnode) load_surf_geo<N, T>(e, own.node, mesh, gm);
+    if (own.active) {
+        load_state<N, T>(e, own.node, U, gd, uc, pr, H);
+        const int pt = Lay<N>::at(own.node);
         s_lift[pt] = pr[1];
         s_lift[n3p + pt] = pr[2];
         s_lift[2 * n3p + pt] = pr[3];
@@ -807,7 +863,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     }
     __syncthreads();
     T g[12];
-    lift_face_fluxes<N, T, TT>(e, tid, mesh, utr, s_lift, s_lflux, gas, nullptr);
+    lift_face_fluxes_packed<N, T, TT>(tid, epb, nElems, mesh, utr, s_buf, s_buf + 4 * n3p, slice, gas, nullptr, 0);
     __syncthreads();
     if (gnode) {
         if constexpr (gradient_in_sequence<N, T>())
@@ -819,7 +875,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     // the stress tensor and heat flux of each surface node (the terms of EvalNormalDiffFlux3D, flux.f90:779-847,
     // before the normal) to its face slots: 9 values per face node instead of the 12 gradients (9 KB less LDS at
     // N=7 in FP64, and FP64 k_lift 4 % faster on MI355X)
-    T* s_q = s_buf + 4 * n3p;  // [6][9][n2]: txx, tyy, tzz, txy, txz, tyz, qx, qy, qz
+    T* s_q = s_lflux;  // [6][9][n2]: txx, tyy, tzz, txy, txz, tyz, qx, qy, qz
     if (gnode) {
         const int pn = Lay<N>::at(gn);
         const T P[4] = {T(0), s_lift[pn], s_lift[n3p + pn], s_lift[2 * n3p + pn]};
@@ -839,11 +895,13 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     __syncthreads();
     // F_v.n_master of each own face node (the index and normal loaded again: cache hits, and no registers held
     // through the gradients)
-    for (int t = tid; t < D::nf; t += D::block) {
-        const FaceTask f = face_task<N>(e, t, mesh);
+    const int nx = Pack<N>::faces(epb, nElems);
+    for (int x = tid; x < nx; x += D::block) {
+        const int le = Pack<N>::face_le(x);
+        const FaceTask f = face_task<N>(Pack<N>::elem(le, epb), x - le * D::nf, mesh);
         const T* fg = GeoOf<T>::fgeo(mesh) + f.side * 10 * n2 + f.pq;
         const T nv[3] = {fg[0], fg[n2], fg[2 * n2]};
-        const T* sq = s_q + (f.ls - 1) * 9 * n2 + f.ab;
+        const T* sq = s_buf + le * slice + 4 * n3p + (f.ls - 1) * 9 * n2 + f.ab;
         T t9[9];
 #pragma unroll
         for (int q = 0; q < 9; q++) t9[q] = sq[q * n2];
@@ -1034,7 +1092,7 @@ struct RhsWaves {
 
 template <int N, typename T, typename TT, bool SPLIT, int RIEMANN>
 __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>::value))
-    k_rhs(const double* U, double* Uout, Mesh mesh, const TT* __restrict__ utr, const TT* __restrict__ vtr,
+    k_rhs(int epb, int nElems, const double* U, double* Uout, Mesh mesh, const TT* __restrict__ utr, const TT* __restrict__ vtr,
           TT* __restrict__ utr_next, double* __restrict__ Ut, double* __restrict__ Kreg, const T* __restrict__ mats,
           GasD gd, T LHm, T LHp, Stage st)
 {
@@ -1060,15 +1118,19 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
     constexpr bool pair_lines = SPLIT && 64 % n == 0 && 64 % n2 == 0;
     constexpr int w_ac = w_a > w_c ? w_a : w_c;
     constexpr int lds_w = w_ac > w_d ? w_ac : w_d;
-    __shared__ T s_w[lds_w];
-    __shared__ T s_geo[geo_lds ? 9 * n3p : 1];  // [3 directions][3][n3p] metrics Ja^1, Ja^2, Ja^3
-    __shared__ T s_nb[6 * 5 * n2];  // neighbour trace records, from the lifting to the face tasks
+    constexpr int most = Pack<N>::most;
+    __shared__ T s_wa[most * lds_w];
+    __shared__ T s_geoa[geo_lds ? most * 9 * n3p : 1];  // [3 directions][3][n3p] metrics Ja^1, Ja^2, Ja^3
+    __shared__ T s_nba[most * 6 * 5 * n2];  // neighbour trace records, from the lifting to the face tasks
     __shared__ Mats<N, T> M;
     __shared__ T s_dp[pair_lines ? n2 : 1];  // DVolSurf by cyclic shift for the shared pairs
-    const int e = blockIdx.x, tid = threadIdx.x;
-    const bool active = tid < n3;
-    const int i = tid % n, j = (tid / n) % n, k = tid / n2;
-    const int pt = Lay<N>::at(tid);
+    const int tid = threadIdx.x;
+    const Pack<N> own(tid, epb, nElems);
+    const int e = own.e, node = own.node;
+    const bool active = own.active;
+    T *s_w = s_wa + own.le * lds_w, *s_geo = s_geoa + (geo_lds ? own.le * 9 * n3p : 0);  // the slices of its element
+    const int i = node % n, j = (node / n) % n, k = node / n2;
+    const int pt = Lay<N>::at(node);
     load_mats<N, T>(M, mats, tid, D::block);
     if (pair_lines && tid < n2) {
         const int sh = tid / n, a = tid % n;
@@ -1084,8 +1146,8 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
     constexpr bool geo_reg = SPLIT && sizeof(T) == 8;
     T gm[10];
     if (active) {
-        if (pgeo) load_node_geo<N, T>(e, tid, mesh, gm);
-        load_state<N, T>(e, tid, U, gd, uc, pr, Hme);
+        if (pgeo) load_node_geo<N, T>(e, node, mesh, gm);
+        load_state<N, T>(e, node, U, gd, uc, pr, Hme);
         if (geo_lds) {
 #pragma unroll
             for (int c = 0; c < 9; c++) s_geo[c * n3p + pt] = T(0.5) * gm[c];  // halves: see the split loop
@@ -1099,24 +1161,24 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
     Stress<T> s;
     {
         T g[12];
-        lift_face_fluxes<N, T, TT>(e, tid, mesh, utr, s_w, s_w + 4 * n3p, gas, s_nb);
+        lift_face_fluxes_packed<N, T, TT>(tid, epb, nElems, mesh, utr, s_wa, s_wa + 4 * n3p, lds_w, gas, s_nba, 30 * n2);
         __syncthreads();
         if (active) {
-            if (!pgeo) load_node_geo<N, T>(e, tid, mesh, gm);
+            if (!pgeo) load_node_geo<N, T>(e, node, mesh, gm);
             if constexpr (mfma_lift)
                 node_gradient_mfma<T>(tid, M, s_w, s_w + 4 * n3p, s_w + w_a0, LHm, LHp, gm, g);
             else if constexpr (gradient_in_sequence<N, T>())
-                node_gradient_seq<N, T>(tid, M, s_w, s_w + 4 * n3p, LHm, LHp, gm, g);
+                node_gradient_seq<N, T>(node, M, s_w, s_w + 4 * n3p, LHm, LHp, gm, g);
             else
-                node_gradient<N, T, Mats<N, T>, lean>(tid, M, s_w, s_w + 4 * n3p, LHm, LHp, gm, g);
+                node_gradient<N, T, Mats<N, T>, lean>(node, M, s_w, s_w + 4 * n3p, LHm, LHp, gm, g);
             stress(pr, g, gas, s);
         }
     }
     __syncthreads();
 
     T ut[5] = {0, 0, 0, 0, 0};
-    const double* ge = mesh.geo + (long)e * 10 * n3 + tid;  // FP64 sJ of the update
-    const T* geT = GeoOf<T>::geo(mesh) + (long)e * 10 * n3 + tid;
+    const double* ge = mesh.geo + (long)e * 10 * n3 + node;  // FP64 sJ of the update
+    const T* geT = GeoOf<T>::geo(mesh) + (long)e * 10 * n3 + node;
     if (!SPLIT) {
         // ---- full transformed fluxes, weak-form D_Hat_T contraction (VolInt_weakForm) ----
         T* s_f = s_w;  // [5][n3p]
@@ -1311,8 +1373,11 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
     }
 
     // ---- face fluxes (FillFlux) and surface integral (SurfInt_Device) ----
-    T* s_res = s_w;  // [6][5][n2]
-    for (int t = tid; t < D::nf; t += D::block) {
+    const int nx = Pack<N>::faces(epb, nElems);
+    for (int x = tid; x < nx; x += D::block) {
+        const int le = Pack<N>::face_le(x), t = x - le * D::nf, e = Pack<N>::elem(le, epb);
+        T* s_res = s_wa + le * lds_w;  // [6][5][n2]
+        const T* s_nb = s_nba + le * 30 * n2;
         int ls = t / n2 + 1, ab = t - (ls - 1) * n2, a = ab % n, b = ab / n;
         int node = face_vol_node<N>(ls, a, b);
         int c = mesh.conn[e * 6 + ls - 1];
@@ -1372,14 +1437,14 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
             if (!on_face<N>(ls, i, j, k, ab)) continue;
             T LH = (ls == 1 || ls == 2 || ls == 5) ? LHm : LHp;
 #pragma unroll
-            for (int v = 0; v < 5; v++) loc[v] = loc[v] + s_res[(ls - 1) * 5 * n2 + v * n2 + ab] * LH;
+            for (int v = 0; v < 5; v++) loc[v] = loc[v] + s_w[(ls - 1) * 5 * n2 + v * n2 + ab] * LH;
         }
-        double* ut_out = (st.mode == 0 ? Ut : Kreg) + (long)e * 5 * n3 + tid;
-        double* un = Uout + (long)e * 5 * n3 + tid;
+        double* ut_out = (st.mode == 0 ? Ut : Kreg) + (long)e * 5 * n3 + node;
+        double* un = Uout + (long)e * 5 * n3 + node;
         double kv[5] = {0, 0, 0, 0, 0}, uv[5] = {0, 0, 0, 0, 0};
         const double sJd = geo_reg ? double(gm[9]) : ge[9 * n3];
         if (st.mode != 0) {
-            const double* uo = U + (long)e * 5 * n3 + tid;
+            const double* uo = U + (long)e * 5 * n3 + node;
             if (st.mRKA != 0.0) {
 #pragma unroll
                 for (int v = 0; v < 5; v++) kv[v] = ut_out[v * n3];
@@ -1417,7 +1482,9 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
         }
     }
     __syncthreads();
-    for (int t = tid; t < D::nf; t += D::block) {
+    for (int x = tid; x < nx; x += D::block) {
+        const int le = Pack<N>::face_le(x), t = x - le * D::nf, e = Pack<N>::elem(le, epb);
+        const T* s_u = s_wa + le * lds_w;
         int ls = t / n2 + 1, ab = t - (ls - 1) * n2;
         int c = mesh.conn[e * 6 + ls - 1];
         long side = c >> 3;
