@@ -28,24 +28,32 @@ struct PrimBar {
 
 __device__ __forceinline__ void prim_bar_zero(PrimBar& b) { b.rho = b.u = b.v = b.w = b.p = b.H = b.T = b.E = 0.0; }
 
-// transposed Jacobian of ConsToPrim (eos.f90:212-239) with H = (E+p)/rho and T = p/(rho*R); rR = 1/R
-__device__ __forceinline__ void prim_bar_to_cons(const double* c, const PrimBar& b, double kappa, double rR,
+// transposed Jacobian of ConsToPrim (eos.f90:212-239) with H = (E+p)/rho and T = p/(rho*R), at the primitive state
+// pr = (rho,u,v,w,p,T) with its H; rR = 1/R
+__device__ __forceinline__ void prim_bar_to_cons(const double* pr, double H, const PrimBar& b, double kappa, double rR,
                                                  double* Ubar)
 {
-    double rho = c[0], sRho = rcp64(rho);
-    double u = c[1] * sRho, v = c[2] * sRho, w = c[3] * sRho;
-    double q2 = 0.5 * (u * u + v * v + w * w);
-    double km1 = kappa - 1.0;
-    double p = km1 * (c[4] - rho * q2);
-    double H = (c[4] + p) * sRho, T = p * sRho * rR;
-    double dp_drho = km1 * q2;
+    const double sRho = rcp64(pr[0]), u = pr[1], v = pr[2], w = pr[3];
+    const double km1 = kappa - 1.0;
+    const double dp_drho = km1 * 0.5 * (u * u + v * v + w * w);
     Ubar[0] = b.rho - (b.u * u + b.v * v + b.w * w) * sRho + b.p * dp_drho + b.H * (dp_drho - H) * sRho +
-              b.T * (dp_drho * sRho * rR - T * sRho);
+              b.T * (dp_drho * rR - pr[5]) * sRho;
     double s = -km1 * (b.p + b.H * sRho + b.T * sRho * rR);
     Ubar[1] = b.u * sRho + s * u;
     Ubar[2] = b.v * sRho + s * v;
     Ubar[3] = b.w * sRho + s * w;
     Ubar[4] = b.E + b.p * km1 + b.H * kappa * sRho + b.T * km1 * sRho * rR;
+}
+
+// the same at the conservative state c
+__device__ __forceinline__ void prim_bar_to_cons(const double* c, const PrimBar& b, double kappa, double rR,
+                                                 double* Ubar)
+{
+    const double sRho = rcp64(c[0]);
+    double pr[6] = {c[0], c[1] * sRho, c[2] * sRho, c[3] * sRho, 0.0, 0.0};
+    pr[4] = (kappa - 1.0) * (c[4] - 0.5 * (c[1] * pr[1] + c[2] * pr[2] + c[3] * pr[3]));
+    pr[5] = pr[4] * sRho * rR;
+    prim_bar_to_cons(pr, (c[4] + pr[4]) * sRho, b, kappa, rR, Ubar);
 }
 
 // Adjoint of the viscous flux -m.(tau, tau.u + lambda grad T) (EvalNormalDiffFlux3D flux.f90:779-847 for m = n,
@@ -336,16 +344,23 @@ __global__ void __launch_bounds__(Dm<N>::block)
 // k_adj_main (split PI volume flux, LF surface flux, FP64)
 //   in : U, U trace records utr (of this U), lam, mu traces; accumulate: Ubar += result, else Ubar = result
 //   out: Ubar, nghtr [side][2][4][n2] = L_Hat(locSide) * (n_master . sJ*Gbar) of the writer
-// Phases: split volume adjoint, forward lifting with the viscous volume adjoint, face adjoint, lifting adjoint.
+// Phases: forward lifting with the viscous volume adjoint, face adjoint, lifting adjoint, split volume adjoint.
+// Bound by latency at the waves in flight, whose number the registers set at N = 5 and 7 and the LDS elsewhere.  The
+// split phase comes last and the faces return their adjoint in primitive form, so that next to nothing of
+// the primitive adjoint is held through the lifting and the faces, and one transposed Jacobian per node takes it all.
+// With the split phase first and a Jacobian per face node the kernel needed 142 registers at N = 5 (now 125: four
+// instead of three workgroups per CU) and spilled 60 bytes per lane at N = 7 (now 20).  us per stage of the reverse
+// sweep before -> now: N = 3, 24^3 elements 242 -> 219; N = 4, 20^3 257 -> 244; N = 5, 16^3 205 -> 181; N = 6, 14^3
+// 305 -> 283; N = 7, 16^3 461 -> 421; N = 8, 12^3 328 -> 317.
 // LDS: one work array reused by the phases, mu = -sJ*lam, the own stress at the face nodes and the matrices
 // (76.5 KB at N=7: two workgroups per CU, with AdjWaves capping the registers to match).
 // ---------------------------------------------------------------------------------------------------------
 template <int N>
 struct AdjLds {
     static constexpr int n2 = Dm<N>::n2, n3 = Dm<N>::n3;
-    static constexpr int w_a = 9 * n3;               // split adjoint partner data: rho,u,v,w,p,H + metric
+    static constexpr int w_a = 8 * n3;               // split adjoint partner data: rho,u,v,w,H + metric
     static constexpr int w_b = 4 * Lay<N>::n3 + 6 * 7 * n2;  // forward lifting (padded layout); also >= 4 n3
-    static constexpr int w_d = 6 * 12 * n2;          // face adjoint results
+    static constexpr int w_d = 6 * 8 * n2;           // face adjoint results
     static constexpr int w_ab = w_a > w_b ? w_a : w_b;
     static constexpr int w = w_ab > w_d ? w_ab : w_d;
     static constexpr int bytes = 8 * (w + 5 * n3 + 6 * 6 * n2 + 3 * Lay<N>::np * (N + 1));  // + Mats
@@ -380,120 +395,26 @@ __global__ void __launch_bounds__(Dm<N>::block, (AdjWaves<N>::value))
     const int i = tid % n, j = (tid / n) % n, k = tid / n2;
     load_mats<N, double, false>(M, mats, tid, D::block);
     const Gas<double> gas = make_gas<double>(gd);
-    double pr[6] = {1, 0, 0, 0, 1, 1};
     const double* ge = mesh.geo + (long)e * 10 * n3 + tid;
     // the node's metrics and sJ are read in each of the three phases that use them: read once into registers
-    // instead, they made the VJP 17 % slower at N=7 on MI355X (the kernel, at 128 VGPRs, spilled 172 instead of 76
-    // bytes per lane)
+    // instead, they made the VJP 17 % slower at N=7 on MI355X, with the split phase first (96 bytes
+    // per lane more in spills)
     PrimBar pb;
     prim_bar_zero(pb);
-    // ---- adjoint of the split volume flux (VolInt_splitForm_Kernel): X(i) += sum_l DVS(l,i) F#(i,l) with F#
-    // symmetric, so U_i receives dF#(i,l)/dU_i^T [DVS(l,i) mu_i + DVS(i,l) mu_l] ----
-    {
-        double* s_v = s_w;           // rho,u,v,w,p,H
-        double* s_m = s_w + 6 * n3;  // metric of the current direction
-        double Hme = 0.0;
-        if (active) {
-            double uc[5];
-            load_state<N, double>(e, tid, U, gd, uc, pr, Hme);
-            s_v[tid] = pr[0];
-            s_v[n3 + tid] = pr[1];
-            s_v[2 * n3 + tid] = pr[2];
-            s_v[3 * n3 + tid] = pr[3];
-            s_v[4 * n3 + tid] = pr[4];
-            s_v[5 * n3 + tid] = Hme;
-            double msJ = -ge[9 * n3];
-            const double* l = lam + (long)e * 5 * n3 + tid;
-#pragma unroll
-            for (int v = 0; v < 5; v++) s_mu[v * n3 + tid] = msJ * l[v * n3];
-        }
-#pragma unroll 1
-        for (int d = 0; d < 3; d++) {
-            double mme[3] = {0, 0, 0};
-            if (active) {
-#pragma unroll
-                for (int c = 0; c < 3; c++) mme[c] = ge[(3 * (d) + (c)) * n3];
-                s_m[tid] = mme[0];
-                s_m[n3 + tid] = mme[1];
-                s_m[2 * n3 + tid] = mme[2];
-            }
-            line_sync<N>(d);  // s_v, s_mu and s_m are read along the lines of d
-            if (active) {
-                int idx = d == 0 ? i : (d == 1 ? j : k);
-                int stride = d == 0 ? 1 : (d == 1 ? n : n2);
-                int base = tid - idx * stride;
-                // the increment of the primitive adjoint (rho,u,v,w,p,H) of pair (idx, l).  F# depends on the
-                // two states only through their sums and the metric sums, so both nodes of the pair receive the
-                // same increment (wv, and with it everything below, is symmetric in the pair)
-                auto pair_bar = [&](int l, double* P) {
-                    const int o = base + l * stride;
-                    const double dli = M.dvs(l, idx), dil = M.dvs(idx, l);
-                    double wv[5];
-#pragma unroll
-                    for (int v = 0; v < 5; v++) wv[v] = dli * s_mu[v * n3 + tid] + dil * s_mu[v * n3 + o];
-                    double sr = pr[0] + s_v[o], su = pr[1] + s_v[n3 + o], sv = pr[2] + s_v[2 * n3 + o],
-                           sw = pr[3] + s_v[3 * n3 + o], sH = Hme + s_v[5 * n3 + o];
-                    double m0 = mme[0] + s_m[o], m1 = mme[1] + s_m[n3 + o], m2 = mme[2] + s_m[2 * n3 + o];
-                    double ms = m0 * su + m1 * sv + m2 * sw;
-                    double q = 0.125 * sr * ms;
-                    double A = 2.0 * wv[0] + su * wv[1] + sv * wv[2] + sw * wv[3] + sH * wv[4];
-                    double c8 = 0.125 * sr * A;
-                    P[0] = 0.125 * ms * A;
-                    P[1] = c8 * m0 + q * wv[1];
-                    P[2] = c8 * m1 + q * wv[2];
-                    P[3] = c8 * m2 + q * wv[3];
-                    P[4] = 0.5 * (m0 * wv[1] + m1 * wv[2] + m2 * wv[3]);
-                    P[5] = q * wv[4];
-                };
-                auto add_bar = [&](const double* P) {
-                    pb.rho += P[0];
-                    pb.u += P[1];
-                    pb.v += P[2];
-                    pb.w += P[3];
-                    pb.p += P[4];
-                    pb.H += P[5];
-                };
-                if (pair_lines && d < 2) {
-                    // lines inside one wave, as the forward's shared pairs: the lane at line position idx forms
-                    // the pairs (idx, idx+s) for s = 1..(n-1)/2 (mod n) and takes (idx-s, idx) from the lane s
-                    // positions back; for even n both ends form (idx, idx+n/2).  The diagonal is left out, as in
-                    // the forward's shared pairs.
-                    constexpr int msk = n - 1;
-                    const int lane0 = (tid & 63) - idx * stride;  // node = thread: lane distance = node stride
-#pragma unroll
-                    for (int s = 1; s <= n / 2; s++) {
-                        double P[6];
-                        pair_bar((idx + s) & msk, P);
-                        add_bar(P);
-                        if (2 * s < n) {
-                            const int src = lane0 + ((idx - s) & msk) * stride;
-                            double R[6];
-#pragma unroll
-                            for (int c = 0; c < 6; c++) R[c] = __shfl(P[c], src);
-                            add_bar(R);
-                        }
-                    }
-                } else {
-                    // l = idx included: F#(U,U) has equal partial derivatives in its two arguments, so the same
-                    // formula gives 2 DVS(i,i) dF#/dU_i^T mu_i.  The forward leaves this pair out; DVS(i,i) is a
-                    // rounding residue for Gauss-Lobatto, so the term is at rounding level either way, and the loop
-                    // over all l spills 8 to 16 bytes per lane less than one that skips it.
-                    for (int l = 0; l <= N; l++) {
-                        double P[6];
-                        pair_bar(l, P);
-                        add_bar(P);
-                    }
-                }
-            }
-            line_sync<N>(d);
-        }
-    }
+    double vel[3] = {0, 0, 0};
     // ---- forward lifting, then the adjoint of the weak viscous volume term (VolInt_weakForm_Visc,
     // volint.f90:60-119): X(i) += sum_l D_Hat_T(l,i) f_d(l)  ->  fbar_d(l) = sum_m D_Hat_T(l,m) mu(m) ----
     ViscGradBar gb;
     visc_grad_zero(gb);
     {
+        double pr[6] = {1, 0, 0, 0, 1, 1};
         if (active) {
+            double uc[5], H;
+            load_state<N, double>(e, tid, U, gd, uc, pr, H);
+            const double msJ = -ge[9 * n3];
+            const double* l = lam + (long)e * 5 * n3 + tid;
+#pragma unroll
+            for (int v = 0; v < 5; v++) s_mu[v * n3 + tid] = msJ * l[v * n3];
             const int pt = Lay<N>::at(tid);  // the lifting reads its input in the padded node layout
             s_w[pt] = pr[1];
             s_w[n3p + pt] = pr[2];
@@ -515,6 +436,9 @@ __global__ void __launch_bounds__(Dm<N>::block, (AdjWaves<N>::value))
 #pragma unroll
                 for (int q = 0; q < 6; q++) o[q * n2] = tau[q];
             }
+            vel[0] = pr[1];
+            vel[1] = pr[2];
+            vel[2] = pr[3];
             double uvw[3] = {0, 0, 0};
 #pragma unroll 1
             for (int d = 0; d < 3; d++) {
@@ -539,7 +463,9 @@ __global__ void __launch_bounds__(Dm<N>::block, (AdjWaves<N>::value))
     __syncthreads();
     // ---- adjoint of the face fluxes (FillFlux fillflux.f90:45-172 + SurfInt_Device surfint.t90:352-586):
     // X(master node) += L_Hat F, X(slave node) -= L_Hat F  ->  Fbar = L_Hat mu_master - L_Hat mu_slave ----
-    double* s_r = s_w;  // [6][12][n2]: Ubar(5), the viscous flux cotangent (4) and the normal (3) of a face node
+    // results of a face node: its primitive adjoint (6) in the slots its stress came from, the direct E part, the
+    // viscous flux cotangent (4) and the normal (3) in s_r
+    double* s_r = s_w;  // [6][8][n2]
     for (int t = tid; t < D::nf; t += D::block) {
         int ls = t / n2 + 1, ab = t - (ls - 1) * n2, a2 = ab % n, b2 = ab / n;
         int node = face_vol_node<N>(ls, a2, b2);
@@ -584,18 +510,18 @@ __global__ void __launch_bounds__(Dm<N>::block, (AdjWaves<N>::value))
         fp.u += uvw[0];
         fp.v += uvw[1];
         fp.w += uvw[2];
-        double Ub[5];
-        prim_bar_to_cons(Uo, fp, gd.kappa, gd.rR, Ub);
-        double* o = s_r + (ls - 1) * 12 * n2 + ab;
+        const double P[6] = {fp.rho, fp.u, fp.v, fp.w, fp.p, fp.H};
+        double* op = s_tau + (ls - 1) * 6 * n2 + ab;
 #pragma unroll
-        for (int v = 0; v < 5; v++) o[v * n2] = Ub[v];
+        for (int q = 0; q < 6; q++) op[q * n2] = P[q];
+        double* o = s_r + (ls - 1) * 8 * n2 + ab;
+        o[0] = fp.E;
 #pragma unroll
-        for (int v = 1; v < 5; v++) o[(4 + v) * n2] = 0.5 * A[v];
+        for (int v = 1; v < 5; v++) o[v * n2] = 0.5 * A[v];
 #pragma unroll
-        for (int d = 0; d < 3; d++) o[(9 + d) * n2] = nv[d];
+        for (int d = 0; d < 3; d++) o[(5 + d) * n2] = nv[d];
     }
     __syncthreads();
-    double Ubf[5] = {0, 0, 0, 0, 0};
     double qb[4] = {0, 0, 0, 0};
     double Gb[12];
     if (active) {
@@ -603,11 +529,17 @@ __global__ void __launch_bounds__(Dm<N>::block, (AdjWaves<N>::value))
         for (int ls = 1; ls <= 6; ls++) {
             int ab;
             if (!on_face<N>(ls, i, j, k, ab)) continue;
-            const double* o = s_r + (ls - 1) * 12 * n2 + ab;
-#pragma unroll
-            for (int v = 0; v < 5; v++) Ubf[v] += o[v * n2];
-            double nv[3] = {o[9 * n2], o[10 * n2], o[11 * n2]};
-            visc_grad_adjoint(pr[1], pr[2], pr[3], nv, o[5 * n2], o[6 * n2], o[7 * n2], o[8 * n2], gb);
+            const double* op = s_tau + (ls - 1) * 6 * n2 + ab;
+            pb.rho += op[0];
+            pb.u += op[n2];
+            pb.v += op[2 * n2];
+            pb.w += op[3 * n2];
+            pb.p += op[4 * n2];
+            pb.H += op[5 * n2];
+            const double* o = s_r + (ls - 1) * 8 * n2 + ab;
+            pb.E += o[0];
+            double nv[3] = {o[5 * n2], o[6 * n2], o[7 * n2]};
+            visc_grad_adjoint(vel[0], vel[1], vel[2], nv, o[n2], o[2 * n2], o[3 * n2], o[4 * n2], gb);
         }
         // ghat = sJ*Gbar: adjoint of g = sJ*(...) in lift_gradient
         visc_grad_expand(gb, gd.mu, gd.lambda, Gb);
@@ -625,8 +557,8 @@ __global__ void __launch_bounds__(Dm<N>::block, (AdjWaves<N>::value))
             long side = c >> 3;
             int flip = c & 7;
             int pq = mesh.inv[(flip * 6 + ls - 1) * n2 + ab];
-            const double* o = s_r + (ls - 1) * 12 * n2 + ab;
-            double nv[3] = {o[9 * n2], o[10 * n2], o[11 * n2]};
+            const double* o = s_r + (ls - 1) * 8 * n2 + ab;
+            double nv[3] = {o[5 * n2], o[6 * n2], o[7 * n2]};
             double se = mesh.fgeo[side * 10 * n2 + 9 * n2 + pq];
             double LH = lhat_of(ls, LHm, LHp);
             double f = flip ? 0.5 * se : -0.5 * se;
@@ -663,24 +595,114 @@ __global__ void __launch_bounds__(Dm<N>::block, (AdjWaves<N>::value))
         }
         line_sync<N>(d);
     }
-    if (!active) return;
     pb.u += qb[0];
     pb.v += qb[1];
     pb.w += qb[2];
     pb.T += qb[3];
-    // U read again: kept in registers since the load (the primitives), it spilled 32 more bytes per lane and
-    // measured 3 % slower on MI355X
-    double cU[5];
-    const double* u = U + (long)e * 5 * n3 + tid;
+    // the state once more: held from the first phase it would cost 14 registers through all phases
+    double pr[6] = {1, 0, 0, 0, 1, 1}, Hme = 0.0;
+    // ---- adjoint of the split volume flux (VolInt_splitForm_Kernel): X(i) += sum_l DVS(l,i) F#(i,l) with F#
+    // symmetric, so U_i receives dF#(i,l)/dU_i^T [DVS(l,i) mu_i + DVS(i,l) mu_l] ----
+    {
+        double* s_v = s_w;           // rho,u,v,w,H
+        double* s_m = s_w + 5 * n3;  // metric of the current direction
+        if (active) {
+            double uc[5];
+            load_state<N, double>(e, tid, U, gd, uc, pr, Hme);
+            s_v[tid] = pr[0];
+            s_v[n3 + tid] = pr[1];
+            s_v[2 * n3 + tid] = pr[2];
+            s_v[3 * n3 + tid] = pr[3];
+            s_v[4 * n3 + tid] = Hme;
+        }
+#pragma unroll 1
+        for (int d = 0; d < 3; d++) {
+            double mme[3] = {0, 0, 0};
+            if (active) {
 #pragma unroll
-    for (int v = 0; v < 5; v++) cU[v] = u[v * n3];
+                for (int c = 0; c < 3; c++) mme[c] = ge[(3 * (d) + (c)) * n3];
+                s_m[tid] = mme[0];
+                s_m[n3 + tid] = mme[1];
+                s_m[2 * n3 + tid] = mme[2];
+            }
+            line_sync<N>(d);  // s_v and s_m are read along the lines of d
+            if (active) {
+                int idx = d == 0 ? i : (d == 1 ? j : k);
+                int stride = d == 0 ? 1 : (d == 1 ? n : n2);
+                int base = tid - idx * stride;
+                // the increment of the primitive adjoint (rho,u,v,w,p,H) of pair (idx, l).  F# depends on the
+                // two states only through their sums and the metric sums, so both nodes of the pair receive the
+                // same increment (wv, and with it everything below, is symmetric in the pair)
+                auto pair_bar = [&](int l, double* P) {
+                    const int o = base + l * stride;
+                    const double dli = M.dvs(l, idx), dil = M.dvs(idx, l);
+                    double wv[5];
+#pragma unroll
+                    for (int v = 0; v < 5; v++) wv[v] = dli * s_mu[v * n3 + tid] + dil * s_mu[v * n3 + o];
+                    double sr = pr[0] + s_v[o], su = pr[1] + s_v[n3 + o], sv = pr[2] + s_v[2 * n3 + o],
+                           sw = pr[3] + s_v[3 * n3 + o], sH = Hme + s_v[4 * n3 + o];
+                    double m0 = mme[0] + s_m[o], m1 = mme[1] + s_m[n3 + o], m2 = mme[2] + s_m[2 * n3 + o];
+                    double ms = m0 * su + m1 * sv + m2 * sw;
+                    double q = 0.125 * sr * ms;
+                    double A = 2.0 * wv[0] + su * wv[1] + sv * wv[2] + sw * wv[3] + sH * wv[4];
+                    double c8 = 0.125 * sr * A;
+                    P[0] = 0.125 * ms * A;
+                    P[1] = c8 * m0 + q * wv[1];
+                    P[2] = c8 * m1 + q * wv[2];
+                    P[3] = c8 * m2 + q * wv[3];
+                    P[4] = 0.5 * (m0 * wv[1] + m1 * wv[2] + m2 * wv[3]);
+                    P[5] = q * wv[4];
+                };
+                auto add_bar = [&](const double* P) {
+                    pb.rho += P[0];
+                    pb.u += P[1];
+                    pb.v += P[2];
+                    pb.w += P[3];
+                    pb.p += P[4];
+                    pb.H += P[5];
+                };
+                if (pair_lines && d < 2) {
+                    // lines inside one wave, as the forward's shared pairs: the lane at line position idx forms
+                    // the pairs (idx, idx+s) for s = 1..(n-1)/2 (mod n) and takes (idx-s, idx) from the lane s
+                    // positions back; for even n both ends form (idx, idx+n/2).  The diagonal is left out, as in
+                    // the forward's shared pairs.
+                    constexpr int msk = n - 1;
+                    const int lane0 = (tid & 63) - idx * stride;  // node = thread: lane distance = node stride
+#pragma unroll 1
+                    for (int s = 1; s <= n / 2; s++) {
+                        double P[6];
+                        pair_bar((idx + s) & msk, P);
+                        add_bar(P);
+                        if (2 * s < n) {
+                            const int src = lane0 + ((idx - s) & msk) * stride;
+                            double R[6];
+#pragma unroll
+                            for (int c = 0; c < 6; c++) R[c] = __shfl(P[c], src);
+                            add_bar(R);
+                        }
+                    }
+                } else {
+                    // l = idx included: F#(U,U) has equal partial derivatives in its two arguments, so the same
+                    // formula gives 2 DVS(i,i) dF#/dU_i^T mu_i.  The forward leaves this pair out; DVS(i,i) is a
+                    // rounding residue for Gauss-Lobatto, so the term is at rounding level either way, and the loop
+                    // over all l needs no per-lane branch.
+                    for (int l = 0; l <= N; l++) {
+                        double P[6];
+                        pair_bar(l, P);
+                        add_bar(P);
+                    }
+                }
+            }
+            line_sync<N>(d);
+        }
+    }
+    if (!active) return;
     double Ubv[5];
-    prim_bar_to_cons(cU, pb, gd.kappa, gd.rR, Ubv);
+    prim_bar_to_cons(pr, Hme, pb, gd.kappa, gd.rR, Ubv);
     double* ub = Ubar + (long)e * 5 * n3 + tid;
 #pragma unroll
     for (int v = 0; v < 5; v++) {
-        double r = Ubv[v] + Ubf[v];
-        ub[v * n3] = accumulate ? ub[v * n3] + r : r;
+        ub[v * n3] = accumulate ? ub[v * n3] + Ubv[v] : Ubv[v];
     }
 }
 
