@@ -164,9 +164,10 @@ int galx_rhs_vjp_device(galx_ctx *ctx, const double *dLam, double *dUbar);
  * final state. */
 int galx_lserk_forward_ckpt(galx_ctx *ctx, double t, double dt, int nSteps, int ckptEvery);
 /* galx_set_adjoint_storage: what the reverse sweep keeps between checkpoints, with C = min(ckptEvery, nSteps).
- *  GALX_ADJ_STAGES (default): each segment is recomputed once and its 5*C stage inputs are kept (in the FP64 form
- *    with their trace records): device memory ~ (nSteps/ckptEvery + 5*C + 1) copies of U (FP64 form: plus 5*C
- *    trace-record sets of 0.75 U each at N=7).
+ *  GALX_ADJ_STAGES (default): the 5*C stage inputs of one segment are kept (in the FP64 form with their trace
+ *    records); the recorded run itself fills them for the last segment, the sweep recomputes each other segment once:
+ *    device memory ~ (nSteps/ckptEvery + 5*C + 1) copies of U (FP64 form: plus 5*C trace-record sets of 0.75 U each at
+ *    N=7).
  *  GALX_ADJ_STEPS: each segment is recomputed once keeping its C step inputs, and each step's stages are
  *    recomputed before its VJPs (4 more RHS evaluations per step, FP64 trace records recomputed per VJP):
  *    ~ (nSteps/ckptEvery + C + 5) copies of U.  The same VJPs on the same stage inputs: the gradient is bitwise
