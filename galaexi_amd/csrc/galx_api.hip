@@ -1195,7 +1195,8 @@ static int lserk_enqueue(galx_ctx* c, double t0, double dt, int iStep0, int nSte
         for (int stage = 0; stage < 5; stage++) {
             launch_lift(c);
             double mRKA = stage == 0 ? 0.0 : -1.0 * RKA[stage];
-            launch_rhs(c, Stage{mRKA, RKB[stage] * dt, 1}, stage_time(step_time(t0, dt, iStep0 + s), dt, stage));
+            const int dropK = stage == 4 && s + 1 < nSteps;
+            launch_rhs(c, Stage{mRKA, RKB[stage] * dt, 1, dropK}, stage_time(step_time(t0, dt, iStep0 + s), dt, stage));
             c->cur ^= 1;
         }
     HIPCHK(hipGetLastError());
@@ -1491,7 +1492,7 @@ static int record_last_segment(galx_ctx* c, double t0, double dt, int iStep0, in
         void* tro = keep && !last ? (void*)c->stageTr[idx + 1] : c->dUtr[c->cur ^ 1];
         launch_lift(c, Ui, tri);
         const double ts = stage_time(step_time(t0, dt, iStep0 + idx / 5), dt, stage);
-        launch_rhs(c, Stage{stage == 0 ? 0.0 : -1.0 * RKA[stage], RKB[stage] * dt, 1}, ts, Ui, Uo, tri, tro);
+        launch_rhs(c, Stage{stage == 0 ? 0.0 : -1.0 * RKA[stage], RKB[stage] * dt, 1, stage == 4 && !last}, ts, Ui, Uo, tri, tro);
         if (!keep || last) c->cur ^= 1;
     }
     HIPCHK(hipGetLastError());
@@ -1548,7 +1549,7 @@ static void adj_recompute_stage(galx_ctx* c, int step, int stage, int q, const d
     const double mRKA = stage == 0 ? 0.0 : -1.0 * RKA[stage];
     const double ts = stage_time(step_time(c->trajT, c->trajDt, step), c->trajDt, stage);
     launch_lift(c, Ui, c->dUtr[q & 1]);
-    launch_rhs(c, Stage{mRKA, RKB[stage] * c->trajDt, 1}, ts, Ui, Uo, c->dUtr[q & 1], c->dUtr[(q + 1) & 1]);
+    launch_rhs(c, Stage{mRKA, RKB[stage] * c->trajDt, 1, stage == 4}, ts, Ui, Uo, c->dUtr[q & 1], c->dUtr[(q + 1) & 1]);
 }
 
 // reverse sweep with GALX_ADJ_STEPS storage: per segment, the recompute keeps the step inputs; per step, in
@@ -1625,7 +1626,7 @@ static int adj_reverse(galx_ctx* c)
                 launch_lift(c, Ui, tri);
                 double mRKA = stage == 0 ? 0.0 : -1.0 * RKA[stage];
                 const double ts = stage_time(step_time(c->trajT, c->trajDt, s0 + s), c->trajDt, stage);
-                launch_rhs(c, Stage{mRKA, RKB[stage] * c->trajDt, 1}, ts, Ui, Uo, tri, tro);
+                launch_rhs(c, Stage{mRKA, RKB[stage] * c->trajDt, 1, stage == 4}, ts, Ui, Uo, tri, tro);
             }
         c->stagesSeg = seg;
         HIPCHK(hipGetLastError());

@@ -226,6 +226,8 @@ struct Stage {
     double mRKA, bdt;
     int mode;  // 0: write Ut; 1: LSERK register update, K = mRKA*K + Ut; with mRKA = 0 (the first stage of a step, or a
                // register that is zero) K is not read: 40 of the stage's 500 bytes per node
+    int dropK = 0;  // mode 1: do not store K, because the stage that follows in the same call does not read it (the last
+                    // stage of a step before another one): another 40 bytes
 };
 
 // matrices staged in LDS: D_T (transpose of D), D_Hat_T, DVolSurf, all (0:N,0:N); dt(a,b), dht(a,b), dvs(a,b)
@@ -1460,7 +1462,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
                 ut_out[v * n3] = utd;
             } else {
                 double kk = kv[v] * st.mRKA + utd;
-                ut_out[v * n3] = kk;
+                if (!st.dropK) ut_out[v * n3] = kk;
                 unew[v] = uv[v] + kk * st.bdt;
                 un[v * n3] = unew[v];
             }

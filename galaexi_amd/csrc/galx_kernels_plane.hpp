@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(Pl<N>::block, 4)
     for (int v = 0; v < 5; v++) {
         const double kv = st.mRKA != 0.0 ? Kreg[at + v * n3] : 0.0;
         const double kk = kv * st.mRKA + double(ut[v] * T(-1)) * sJ;
-        Kreg[at + v * n3] = kk;
+        if (!st.dropK) Kreg[at + v * n3] = kk;
         unew[v] = U[at + v * n3] + kk * st.bdt;
         Uout[at + v * n3] = unew[v];
     }
