@@ -183,7 +183,8 @@ __global__ void k_grad_to_ref(long nDOF, int n3, int nv, const double* __restric
 // the node's coordinate combination (x+y+z for 4; x, y or z for 41, 42, 43) and the table c built on the host.
 // S is a physical-space rate: the reference adds S/sJ before scaling Ut by sJ, which is S added after it.
 // mode 0 (after the RHS kernel wrote Ut):  X = Ut,  X += S.
-// mode 1 (before an LSERK stage whose RHS kernel then runs with mRKA = 1):  X = K,  X = mRKA*K + S.
+// mode 1 (mixed form, before an LSERK stage whose RHS kernel then runs with mRKA = 1):  X = K,  X = mRKA*K + S.  The FP64
+// form adds the source of a stage in the kernel that updates the register (StageSource).
 struct SourceCoefs {
     double c[5][3];
     double omega, a;
@@ -207,6 +208,14 @@ __global__ void __launch_bounds__(256) k_source(long nDOF, int n3, const double*
         const double o = mode == 0 || mRKA != 0.0 ? p[v * n3] : 0.0;
         p[v * n3] = mode == 0 ? o + S : o * mRKA + S;
     }
+}
+
+// sin and cos of omega*xs of every node: the table of StageSource
+__global__ void __launch_bounds__(256) k_source_table(long nDOF, const double* __restrict__ xs, double omega,
+                                                      double* __restrict__ tab)
+{
+    long x = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (x < nDOF) sincos(omega * xs[x], &tab[x], &tab[nDOF + x]);
 }
 
 // k_ref_to_planes with the per-block sums of the pressure and of the enthalpy H = (E+p)/rho over the nodes (the mixed
@@ -503,6 +512,7 @@ struct galx_ctx {
     int srcFunc = 0;
     SourceCoefs src{};
     double* dSrcX = nullptr;
+    double* dSrcTab = nullptr;  // FP64 form: the table of StageSource
     double* hPsum = nullptr;  // pinned: per-block pressure and enthalpy sums (mixed form's offsets)
     long long bytes = 0;
     bool timing = false;
@@ -860,7 +870,7 @@ int galx_destroy(galx_ctx* c)
                   c->dGeo32,  c->dFgeo32, c->dSgeo32, c->dWs};
     for (void* p : ps) dfree(p);
     void* pa[] = {c->dKbar,    c->dUbar,   c->dMutr,    c->dNghtr, c->dUfinal,
-                  c->dGrad,    c->dGradRef, c->dMats64, c->dTr64,  c->dSrcX};
+                  c->dGrad,    c->dGradRef, c->dMats64, c->dTr64,  c->dSrcX, c->dSrcTab};
     for (void* p : pa) dfree(p);
     for (double* p : c->ckpt) dfree(p);
     for (double* p : c->stages) dfree(p);
@@ -1040,6 +1050,12 @@ int galx_set_source(galx_ctx* c, int exactFunc, const double* advVel, const doub
     int rc;
     if ((rc = dalloc(c, &c->dSrcX, nDOF * sizeof(double)))) return rc;
     HIPCHK(hipMemcpyAsync(c->dSrcX, xs.data(), nDOF * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    if (c->tsz == 8) {
+        if ((rc = dalloc(c, &c->dSrcTab, 2 * nDOF * sizeof(double)))) return rc;
+        k_source_table<<<dim3((unsigned)((nDOF + 255) / 256)), dim3(256), 0, c->stream>>>(nDOF, c->dSrcX, sc.omega,
+                                                                                        c->dSrcTab);
+        HIPCHK(hipGetLastError());
+    }
     HIPCHK(hipStreamSynchronize(c->stream));
     c->src = sc;
     c->srcFunc = exactFunc;
@@ -1107,9 +1123,9 @@ static void launch_source(galx_ctx* c, double t, int mode, double mRKA)
 
 // one RHS pass at time t (the stage time; it enters only through the manufactured source) on the state U
 // (default: the context state) with its traces utr, the updated state to Uout (default: in place) and its
-// traces to utr_next (defaults: the double-buffered context traces).  With a source, an LSERK stage first folds
-// it into the register (K = mRKA*K + S) and the RHS kernel then adds its own rate with mRKA = 1; a plain RHS
-// evaluation adds it to Ut afterwards.
+// traces to utr_next (defaults: the double-buffered context traces).  With a source, the RHS kernel of an FP64 LSERK stage
+// adds it on its way (StageSource); that of a mixed stage runs with mRKA = 1 after the source was folded into the register
+// (K = mRKA*K + S), which leaves its FP32 code alone; a plain RHS evaluation adds it to Ut afterwards.
 static void launch_rhs(galx_ctx* c, Stage st, double t, const double* U = nullptr, double* Uout = nullptr,
                        const void* utr = nullptr, void* utr_next = nullptr)
 {
@@ -1117,7 +1133,14 @@ static void launch_rhs(galx_ctx* c, Stage st, double t, const double* U = nullpt
         if (c->kZero) st.mRKA = 0.0;  // the kernels then leave the register's memory unread
         c->kZero = false;
     }
-    if (c->srcFunc && st.mode == 1) {
+    if (c->srcFunc && st.mode == 1 && c->tsz == 8) {
+        StageSource& q = st.src;
+        q.tab = c->dSrcTab;
+        q.nDOF = (long)c->nElems * c->n3;
+        std::memcpy(q.c, c->src.c, sizeof(q.c));
+        q.sinat = std::sin(c->src.a * t);
+        q.cosat = std::cos(c->src.a * t);
+    } else if (c->srcFunc && st.mode == 1) {
         launch_source(c, t, 1, st.mRKA);
         st.mRKA = 1.0;
     }

@@ -222,12 +222,38 @@ struct GeoOf<float> {
     __device__ static __forceinline__ const float* sgeo(const Mesh& m) { return m.sgeo32; }
 };
 
+// manufactured source of the stage, added to the LSERK register by the kernel that updates it (FP64; null tab: none).
+// S_v = c[v][0] cos(phi) + c[v][1] sin(2 phi) + c[v][2] sin(phi) with phi = omega*xs - a*t: the node's sin and cos of
+// omega*xs from the table, those of a*t from the host, the angle sum here.  A pass of its own over the register moved 80
+// bytes per node and launched once more per stage: five steps at N = 3 on 16^3 elements, CalcTimeStep included, 1734 -> 1628
+// us without it, two at N = 11 on 2^3 418 -> 358 us.  sincos in the kernel instead of the table would bring its
+// large-argument path and the registers of that into every k_rhs.
+struct StageSource {
+    const double* tab;  // sin(omega*xs) of every node, element planes, then cos(omega*xs)
+    long nDOF;
+    double c[5][3];
+    double sinat, cosat;
+};
+
+// k = mRKA*k + S at node x; returns the coefficient k still takes (1; mRKA where there is no source)
+__device__ __forceinline__ double source_into_register(const StageSource& src, long x, double mRKA, double* k)
+{
+    if (!src.tab) return mRKA;
+    const double sx = src.tab[x], cx = src.tab[src.nDOF + x];
+    const double sn = sx * src.cosat - cx * src.sinat, cs = cx * src.cosat + sx * src.sinat, sn2 = 2.0 * sn * cs;
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+        k[v] = k[v] * mRKA + (src.c[v][0] * cs + src.c[v][1] * sn2 + src.c[v][2] * sn);
+    return 1.0;
+}
+
 struct Stage {
     double mRKA, bdt;
     int mode;  // 0: write Ut; 1: LSERK register update, K = mRKA*K + Ut; with mRKA = 0 (the first stage of a step, or a
                // register that is zero) K is not read: 40 of the stage's 500 bytes per node
     int dropK = 0;  // mode 1: do not store K, because the stage that follows in the same call does not read it (the last
                     // stage of a step before another one): another 40 bytes
+    StageSource src{};
 };
 
 // matrices staged in LDS: D_T (transpose of D), D_Hat_T, DVolSurf, all (0:N,0:N); dt(a,b), dht(a,b), dvs(a,b)
@@ -1454,6 +1480,8 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
 #pragma unroll
             for (int v = 0; v < 5; v++) uv[v] = uo[v * n3];
         }
+        double ak = st.mRKA;
+        if (sizeof(T) == 8 && st.mode != 0) ak = source_into_register(st.src, (long)e * n3 + node, ak, kv);
 #pragma unroll
         for (int v = 0; v < 5; v++) {
             T tot = ut[v] + loc[v];
@@ -1461,7 +1489,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
             if (st.mode == 0) {
                 ut_out[v * n3] = utd;
             } else {
-                double kk = kv[v] * st.mRKA + utd;
+                double kk = kv[v] * ak + utd;
                 if (!st.dropK) ut_out[v * n3] = kk;
                 unew[v] = uv[v] + kk * st.bdt;
                 un[v * n3] = unew[v];

@@ -454,11 +454,13 @@ __global__ void __launch_bounds__(Pl<N>::block, 4)
         for (int v = 0; v < 5; v++) Ut[at + v * n3] = double(ut[v] * T(-1)) * sJ;
         return;
     }
-    double unew[5], tr[5];
+    double unew[5], tr[5], kv[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) kv[v] = st.mRKA != 0.0 ? Kreg[at + v * n3] : 0.0;
+    const double ak = source_into_register(st.src, (long)e * n3 + nd.node, st.mRKA, kv);
 #pragma unroll
     for (int v = 0; v < 5; v++) {
-        const double kv = st.mRKA != 0.0 ? Kreg[at + v * n3] : 0.0;
-        const double kk = kv * st.mRKA + double(ut[v] * T(-1)) * sJ;
+        const double kk = kv[v] * ak + double(ut[v] * T(-1)) * sJ;
         if (!st.dropK) Kreg[at + v * n3] = kk;
         unew[v] = U[at + v * n3] + kk * st.bdt;
         Uout[at + v * n3] = unew[v];
