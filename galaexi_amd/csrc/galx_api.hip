@@ -8,11 +8,11 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -653,8 +653,8 @@ struct Staging {
 // this call empty, so that copying and page faults run beside the transfer.  us on MI355X at N = 7, into new arrays: state
 // of 8^3 elements (10.5 MB) 747 -> 520, its gradients (25 MB) 3287 -> 1125 (1809 in another process), state of 16^3
 // (84 MB) 7989 -> 2820; 4.4 MB 334 -> 309; at 2.6 MB as fast as the plain copy.  Chunks of 1 MiB were 25 % slower, 6 or 8
-// threads no faster, 8 slots 16 % faster at 84 MB only, for a longer first call.  Pinned destinations and small ones keep the plain copy, and so does a host that has no memory or
-// threads to give.
+// threads no faster, 8 slots 16 % faster at 84 MB only, for a longer first call.  Pinned destinations and small ones keep
+// the plain copy, and so does a host that has no memory or threads to give.
 struct HostOut {
     double* dst;
     const double* src;
@@ -708,7 +708,7 @@ static int copy_staged(galx_ctx* c, const std::vector<HostOut>& chunks, bool& co
     team.reserve(OUT_THREADS);
     try {
         for (int w = 0; w < OUT_THREADS; w++) team.emplace_back(empty, w, OUT_THREADS);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {  // no thread or no memory for one
         stop.store(true, std::memory_order_release);
         for (auto& t : team) t.join();
         return GALX_OK;  // nothing copied: the plain copy takes over
