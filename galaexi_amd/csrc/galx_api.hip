@@ -306,9 +306,17 @@ struct Launch {
                                    (const T*)utr, (T*)vtr, (const T*)mats, g, T(LHm), T(LHp));
                 return;
             }
-        if constexpr (whole)
-            hipLaunchKernelGGL((k_lift<N, T, T>), pack_grid(nE), dim3(D::block), 0, s, Pack<N>::of(nE),
-                               nE, U, m, (const T*)utr, (T*)vtr, (const T*)mats, g, T(LHm), T(LHp));
+        if constexpr (whole) {
+            constexpr int wide = FaceBlock<N>::value;
+            auto launch = [&](auto kernel, int block) {
+                hipLaunchKernelGGL(kernel, pack_grid(nE), dim3(block), 0, s, Pack<N>::of(nE), nE, U, m, (const T*)utr,
+                                   (T*)vtr, (const T*)mats, g, T(LHm), T(LHp));
+            };
+            if (FaceBlock<N>::template lift<T>(nE))
+                launch(k_lift<N, T, T, wide>, wide);
+            else
+                launch(k_lift<N, T, T>, D::block);
+        }
     }
     template <int RIE>
     static void rhs_r(hipStream_t s, int nE, const double* U, double* Uout, Mesh m, const void* utr, const void* vtr,
@@ -322,10 +330,18 @@ struct Launch {
                                    T(LHm), T(LHp), st);
                 return;
             }
-        if constexpr (whole)
-            hipLaunchKernelGGL((k_rhs<N, T, T, SPLIT, RIE>), pack_grid(nE), dim3(D::block), 0, s,
-                               Pack<N>::of(nE), nE, U, Uout, m, (const T*)utr, (const T*)vtr, (T*)utr_next, Ut, K,
-                               (const T*)mats, g, T(LHm), T(LHp), st);
+        if constexpr (whole) {
+            constexpr int wide = FaceBlock<N>::value;
+            auto launch = [&](auto kernel, int block) {
+                hipLaunchKernelGGL(kernel, pack_grid(nE), dim3(block), 0, s, Pack<N>::of(nE), nE, U, Uout, m,
+                                   (const T*)utr, (const T*)vtr, (T*)utr_next, Ut, K, (const T*)mats, g, T(LHm), T(LHp),
+                                   st);
+            };
+            if (FaceBlock<N>::rhs(nE))
+                launch(k_rhs<N, T, T, SPLIT, RIE, wide>, wide);
+            else
+                launch(k_rhs<N, T, T, SPLIT, RIE>, D::block);
+        }
     }
     static void rhs(hipStream_t s, int nE, const double* U, double* Uout, Mesh m, const void* utr, const void* vtr,
                     void* utr_next, double* Ut, double* K, const void* mats, GasD g, int riemann, double LHm,

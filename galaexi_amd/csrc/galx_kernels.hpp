@@ -81,6 +81,28 @@ struct Pack {
     }
 };
 
+// Threads of a workgroup that take the face nodes of an element in one pass: 96 and 150 of them at N = 3 and 4, where the
+// 64 and 128 threads of the volume nodes need two.  us on MI355X, before -> after:
+//   k_lift in FP64 always runs with them: N = 3 9.1 -> 8.0 at 8^3 elements, 21.0 -> 20.4 at 16^3, 86.5 -> 85.3 at 28^3;
+//   N = 4 11.8 -> 10.9 at 9^3, 31.1 -> 29.7 at 16^3.  Mixed 8.5 -> 7.3 at 8^3, 14.4 -> 13.1 at 16^3, but 47.8 -> 50.3 at
+//   28^3: up to the 16 workgroups per CU that fit beside each other.
+//   k_rhs does on meshes that do not fill the chip: its face task is a longer part of the workgroup's serial chain, but in
+//   the other phases the added wave only waits, and holds registers that another workgroup could use.  N = 3 weak Roe 13.6
+//   -> 11.7 at 8^3, 18.3 -> 16.2 at 11^3, split RoeEntropyFix 22.8 -> 25.2 at 12^3: the line is six workgroups per CU, all
+//   that fit beside each other.  N = 4 split LF 19.0 -> 17.1 at 8^3, 50.3 -> 47.9 at 14^3, weak Roe 59.2 -> 60.4 at 16^3:
+//   twelve per CU.
+template <int N>
+struct FaceBlock {
+    static constexpr bool wider = N == 3 || N == 4;
+    static constexpr int value = wider ? (Dm<N>::nf + 63) / 64 * 64 : Dm<N>::block;
+    template <typename T>
+    static bool lift(int nElems)
+    {
+        return wider && (sizeof(T) == 8 || nElems <= 16 * 256);
+    }
+    static bool rhs(int nElems) { return wider && nElems <= (N == 3 ? 6 : 12) * 256; }
+};
+
 // nodes on the element surface, n^3 - (n-2)^3 of them
 __host__ __device__ constexpr int surface_count(int N) { return 2 * (N + 1) * (N + 1) + (N - 1) * 4 * N; }
 
@@ -397,13 +419,13 @@ __device__ __forceinline__ void lift_face_fluxes(int e, int tid, const Mesh& mes
 }
 
 // the same for the elements of a packed workgroup, whose LDS slices lie `slice` (s_lift, s_lflux) and nb_slice apart
-template <int N, typename T, typename TT>
+template <int N, typename T, typename TT, int BLK>
 __device__ __forceinline__ void lift_face_fluxes_packed(int tid, int epb, int nElems, const Mesh& mesh,
                                                         const TT* __restrict__ utr, const T* s_lift, T* s_lflux,
                                                         int slice, const Gas<T>& gas, T* s_nb, int nb_slice)
 {
     const int nx = Pack<N>::faces(epb, nElems);
-    for (int x = tid; x < nx; x += Dm<N>::block) {
+    for (int x = tid; x < nx; x += BLK) {
         const int le = Pack<N>::face_le(x);
         const FaceTask f = face_task<N>(Pack<N>::elem(le, epb), x - le * Dm<N>::nf, mesh);
         LiftOperands<T> p;
@@ -850,8 +872,8 @@ struct LiftWaves {
     static constexpr int value = (w > 0 && Dm<N>::block >= 256) ? w : 1;
 };
 
-template <int N, typename T, typename TT>
-__global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
+template <int N, typename T, typename TT, int BLK = Dm<N>::block>
+__global__ void __launch_bounds__(BLK, (LiftWaves<N, T>::value))
     k_lift(int epb, int nElems, const double* __restrict__ U, Mesh mesh, const TT* __restrict__ utr, TT* __restrict__ vtr,
            const T* __restrict__ mats, GasD gd, T LHm, T LHp)
 {
@@ -869,7 +891,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     const int e = own.e;
     T* s_lift = s_buf + own.le * slice;
     T* s_lflux = s_lift + 4 * n3p;
-    load_mats<N, T>(M, mats, tid, D::block);
+    load_mats<N, T>(M, mats, tid, BLK);
     const Gas<T> gas = make_gas<T>(gd);
     T uc[5], pr[6], H;
     // only the surface nodes' gradients are used (for F_v.n on the faces): the first Surf<N>::count threads
@@ -891,7 +913,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     }
     __syncthreads();
     T g[12];
-    lift_face_fluxes_packed<N, T, TT>(tid, epb, nElems, mesh, utr, s_buf, s_buf + 4 * n3p, slice, gas, nullptr, 0);
+    lift_face_fluxes_packed<N, T, TT, BLK>(tid, epb, nElems, mesh, utr, s_buf, s_buf + 4 * n3p, slice, gas, nullptr, 0);
     __syncthreads();
     if (gnode) {
         if constexpr (gradient_in_sequence<N, T>())
@@ -924,7 +946,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (LiftWaves<N, T>::value))
     // F_v.n_master of each own face node (the index and normal loaded again: cache hits, and no registers held
     // through the gradients)
     const int nx = Pack<N>::faces(epb, nElems);
-    for (int x = tid; x < nx; x += D::block) {
+    for (int x = tid; x < nx; x += BLK) {
         const int le = Pack<N>::face_le(x);
         const FaceTask f = face_task<N>(Pack<N>::elem(le, epb), x - le * D::nf, mesh);
         const T* fg = GeoOf<T>::fgeo(mesh) + f.side * 10 * n2 + f.pq;
@@ -1118,8 +1140,8 @@ struct RhsWaves {
         sizeof(T) == 8 ? fp64 : (RIEMANN == RIEMANN_ROEEF || Dm<N>::block < 256 ? 1 : GALX_MIXED_WAVES);
 };
 
-template <int N, typename T, typename TT, bool SPLIT, int RIEMANN>
-__global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>::value))
+template <int N, typename T, typename TT, bool SPLIT, int RIEMANN, int BLK = Dm<N>::block>
+__global__ void __launch_bounds__(BLK, (RhsWaves<N, RIEMANN, T, SPLIT>::value))
     k_rhs(int epb, int nElems, const double* U, double* Uout, Mesh mesh, const TT* __restrict__ utr, const TT* __restrict__ vtr,
           TT* __restrict__ utr_next, double* __restrict__ Ut, double* __restrict__ Kreg, const T* __restrict__ mats,
           GasD gd, T LHm, T LHp, Stage st)
@@ -1159,7 +1181,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
     T *s_w = s_wa + own.le * lds_w, *s_geo = s_geoa + (geo_lds ? own.le * 9 * n3p : 0);  // the slices of its element
     const int i = node % n, j = (node / n) % n, k = node / n2;
     const int pt = Lay<N>::at(node);
-    load_mats<N, T>(M, mats, tid, D::block);
+    load_mats<N, T>(M, mats, tid, BLK);
     if (pair_lines && tid < n2) {
         const int sh = tid / n, a = tid % n;
         s_dp[tid] = mats[2 * n2 + ((a + sh) & (n - 1)) + n * a];
@@ -1189,7 +1211,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
     Stress<T> s;
     {
         T g[12];
-        lift_face_fluxes_packed<N, T, TT>(tid, epb, nElems, mesh, utr, s_wa, s_wa + 4 * n3p, lds_w, gas, s_nba, 30 * n2);
+        lift_face_fluxes_packed<N, T, TT, BLK>(tid, epb, nElems, mesh, utr, s_wa, s_wa + 4 * n3p, lds_w, gas, s_nba, 30 * n2);
         __syncthreads();
         if (active) {
             if (!pgeo) load_node_geo<N, T>(e, node, mesh, gm);
@@ -1401,8 +1423,10 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
     }
 
     // ---- face fluxes (FillFlux) and surface integral (SurfInt_Device) ----
+    // at N = 3 the volume terms are ordered by their one wave alone (line_sync): the added wave waits for it here
+    if (BLK > D::block) __syncthreads();
     const int nx = Pack<N>::faces(epb, nElems);
-    for (int x = tid; x < nx; x += D::block) {
+    for (int x = tid; x < nx; x += BLK) {
         const int le = Pack<N>::face_le(x), t = x - le * D::nf, e = Pack<N>::elem(le, epb);
         T* s_res = s_wa + le * lds_w;  // [6][5][n2]
         const T* s_nb = s_nba + le * 30 * n2;
@@ -1512,7 +1536,7 @@ __global__ void __launch_bounds__(Dm<N>::block, (RhsWaves<N, RIEMANN, T, SPLIT>:
         }
     }
     __syncthreads();
-    for (int x = tid; x < nx; x += D::block) {
+    for (int x = tid; x < nx; x += BLK) {
         const int le = Pack<N>::face_le(x), t = x - le * D::nf, e = Pack<N>::elem(le, epb);
         const T* s_u = s_wa + le * lds_w;
         int ls = t / n2 + 1, ab = t - (ls - 1) * n2;
