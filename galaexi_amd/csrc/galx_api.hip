@@ -1669,9 +1669,9 @@ int galx_lserk_forward_ckpt(galx_ctx* c, double t, double dt, int nSteps, int ck
     const int C = std::min(ckptEvery, nSteps);
     const bool keepStages = c->adjStorage == GALX_ADJ_STAGES;
     // storage: checkpoints; GALX_ADJ_STAGES: the stage inputs of one segment, and in the FP64 form their trace
-    // records, kept for the VJPs by this run for the last segment and by the recompute for the others (the mixed form recomputes FP64 records per VJP, its forward
-    // records being FP32); GALX_ADJ_STEPS: the step inputs of one segment and the stage inputs 1..4 of one step,
-    // trace records recomputed per VJP in both forms
+    // records, kept for the VJPs (by this run for the last segment, by the recompute for the others; the mixed form
+    // recomputes FP64 records per VJP, its forward records being FP32); GALX_ADJ_STEPS: the step inputs of one segment
+    // and the stage inputs 1..4 of one step, trace records recomputed per VJP in both forms
     const size_t tb = 2L * 5 * c->nSides * c->n2 * sizeof(double);
     c->trajValid = false;
     c->stagesSeg = -1;
