@@ -4,7 +4,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -489,6 +491,7 @@ struct Timer {
 // copy_to_host: slots and size of its pinned staging, and the threads that empty it
 static constexpr int OUT_SLOTS = 4, OUT_THREADS = 4;
 static constexpr size_t OUT_CHUNK = (size_t)2 << 20;
+static constexpr int OUT_SPIN_US = 200;  // waits within a copy that is under way: a chunk arrives every 40 us
 
 struct galx_ctx {
     galx_config cfg;
@@ -669,8 +672,10 @@ struct Staging {
 // this call empty, so that copying and page faults run beside the transfer.  us on MI355X at N = 7, into new arrays: state
 // of 8^3 elements (10.5 MB) 747 -> 520, its gradients (25 MB) 3287 -> 1125 (1809 in another process), state of 16^3
 // (84 MB) 7989 -> 2820; 4.4 MB 334 -> 309; at 2.6 MB as fast as the plain copy.  Chunks of 1 MiB were 25 % slower, 6 or 8
-// threads no faster, 8 slots 16 % faster at 84 MB only, for a longer first call.  Pinned destinations and small ones keep
-// the plain copy, and so does a host that has no memory or threads to give.
+// threads no faster, 8 slots 16 % faster at 84 MB only, for a longer first call.  The threads sleep until the first chunk
+// arrives, i.e. until the work queued before the call has ended (a host-form reverse sweep of 22 ms took 98 ms of processor
+// time while they spun there, and takes 22), and spin for at most OUT_SPIN_US after that.  Pinned destinations and small
+// ones keep the plain copy, and so does a host that has no memory or threads to give.
 struct HostOut {
     double* dst;
     const double* src;
@@ -706,26 +711,40 @@ static bool pageable(const void* p)
 static int copy_staged(galx_ctx* c, const std::vector<HostOut>& chunks, bool& copied)
 {
     const long n = (long)chunks.size();
-    std::vector<std::atomic<char>> done(n);
+    std::vector<std::atomic<char>> done(n);  // chunks emptied
     for (auto& d : done) d.store(0, std::memory_order_relaxed);
-    std::atomic<long> ready{0};
+    std::atomic<long> ready{0};  // chunks that have arrived in their slots
     std::atomic<bool> stop{false};
-    auto empty = [&](int w, int threads) {
-        for (long i = w; i < n; i += threads) {
-            while (ready.load(std::memory_order_acquire) <= i) {
-                if (stop.load(std::memory_order_acquire)) return;
-                std::this_thread::yield();
-            }
+    std::mutex mx;
+    std::condition_variable changed;
+    auto tell = [&] {
+        { std::lock_guard<std::mutex> lk(mx); }  // a waiter is before its look at the condition or asleep
+        changed.notify_all();
+    };
+    auto wait = [&](bool spin, auto cond) {
+        for (const auto t0 = std::chrono::steady_clock::now(); spin && !cond(); std::this_thread::yield())
+            spin = std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(OUT_SPIN_US);
+        std::unique_lock<std::mutex> lk(mx);
+        changed.wait(lk, cond);
+    };
+    auto empty = [&](int w) {
+        for (long i = w; i < n; i += OUT_THREADS) {
+            // the first chunk comes after all work queued before the call, which may be a reverse sweep of seconds
+            auto here = [&] { return ready.load(std::memory_order_acquire) > i; };
+            wait(i >= OUT_THREADS, [&] { return here() || stop.load(std::memory_order_acquire); });
+            if (!here()) return;
             std::memcpy(chunks[i].dst, c->hStage + (i % OUT_SLOTS) * OUT_CHUNK, chunks[i].bytes);
             done[i].store(1, std::memory_order_release);
+            tell();
         }
     };
     std::vector<std::thread> team;
     team.reserve(OUT_THREADS);
     try {
-        for (int w = 0; w < OUT_THREADS; w++) team.emplace_back(empty, w, OUT_THREADS);
+        for (int w = 0; w < OUT_THREADS; w++) team.emplace_back(empty, w);
     } catch (const std::exception&) {  // no thread or no memory for one
         stop.store(true, std::memory_order_release);
+        tell();
         for (auto& t : team) t.join();
         return GALX_OK;  // nothing copied: the plain copy takes over
     }
@@ -736,7 +755,7 @@ static int copy_staged(galx_ctx* c, const std::vector<HostOut>& chunks, bool& co
             const long before = issued - OUT_SLOTS;  // the chunk that had this slot
             if (before >= 0 && !done[before].load(std::memory_order_acquire)) {
                 if (issued > i) break;  // there is one to wait for on the device first
-                while (!done[before].load(std::memory_order_acquire)) std::this_thread::yield();
+                wait(true, [&] { return done[before].load(std::memory_order_acquire) != 0; });
             }
             const HostOut& o = chunks[issued];
             const int s = (int)(issued % OUT_SLOTS);
@@ -744,9 +763,15 @@ static int copy_staged(galx_ctx* c, const std::vector<HostOut>& chunks, bool& co
             if (e == hipSuccess) e = hipEventRecord(c->stageEv[s], c->stream);
         }
         if (e == hipSuccess) e = hipEventSynchronize(c->stageEv[i % OUT_SLOTS]);
-        if (e == hipSuccess) ready.store(i + 1, std::memory_order_release);
+        if (e == hipSuccess) {
+            ready.store(i + 1, std::memory_order_release);
+            tell();
+        }
     }
-    if (e != hipSuccess) stop.store(true, std::memory_order_release);
+    if (e != hipSuccess) {
+        stop.store(true, std::memory_order_release);
+        tell();
+    }
     for (auto& t : team) t.join();
     HIPCHK(e);
     copied = true;

@@ -1,0 +1,113 @@
+"""The library's host code with the HIP runtime replaced (tests/native/hip_stub.cpp): results on their way to pageable host
+arrays.  Device memory holds the indices of its doubles, and so does the state handed in; no kernel runs, so a result is right
+if it is arange.  A copy that nobody waits for never arrives.  Each scenario runs in a process of its own, with the stub ahead of the HIP runtime."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PRELUDE = """
+import ctypes, sys, time
+import numpy as np
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.modules["torch"] = None  # its HIP runtime would be loaded ahead of the stub
+from galaexi_amd import _lib, dg, mesh as M
+
+def fail(name, nth):
+    stub.stub_fail(name.encode(), ctypes.c_long(nth))
+
+def calls(name):
+    return stub.stub_calls(name.encode())
+
+def context(N, nel, precision="fp64"):
+    op = dg.DGOperator(N, form="split", riemann="lf", precision=precision, mu0=1e-3, R=1.0)
+    m = M.box_mesh(nel, N, lo=(-1.0,) * 3, hi=(1.0,) * 3)
+    op.set_mesh(m)
+    op.set_state(np.arange(5.0 * (N + 1) ** 3 * m.nElems).reshape((5, N + 1, N + 1, N + 1, m.nElems), order="F"))
+    return op
+
+def right(U):
+    return np.array_equal(U.ravel(order="F"), np.arange(U.size))
+
+def refused(f, *a):
+    try:
+        f(*a)
+    except _lib.GalxError as e:
+        return str(e)
+    raise AssertionError("not refused")
+
+CHUNKS = 12  # of 2 MiB, over 4 slots: the results of BIG
+BIG = (4, (11, 21, 21))
+assert 11 * 21 * 21 * 125 * 40 > (CHUNKS - 1) << 21 and 11 * 21 * 21 * 125 * 40 < CHUNKS << 21
+"""
+
+
+@pytest.fixture(scope="session")
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("hip_stub") / "libhip_stub.so")
+    src = os.path.join(ROOT, "tests", "native", "hip_stub.cpp")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-o", out, src], check=True)
+    return out
+
+
+def run(stub, body):
+    env = dict(os.environ, OMP_NUM_THREADS="1", OPENBLAS_NUM_THREADS="1")
+    res = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body), stub], cwd=ROOT, env=env, text=True,
+                         capture_output=True, timeout=100)
+    assert res.returncode == 0, res.stdout + res.stderr
+
+
+needs_cores = pytest.mark.skipif(len(os.sched_getaffinity(0)) <= 4, reason="hosts of few cores take the plain copy")
+
+
+@needs_cores
+def test_large_results_go_through_the_chunks(stub):
+    run(stub, """
+        op = context(*BIG)
+        for _ in range(3):
+            n = calls("hipMemcpyAsync")
+            assert right(op.get_state())
+            assert calls("hipMemcpyAsync") - n == CHUNKS
+        op.close()
+        op = context(4, (10, 9, 9))  # 4.05 MB, below 4 MiB: one plain copy
+        n = calls("hipMemcpyAsync")
+        assert right(op.get_state()) and calls("hipMemcpyAsync") - n == 1
+    """)
+
+
+@needs_cores
+def test_waiting_for_queued_work_takes_no_processor_time(stub):
+    """Copies start when the work queued before them is done; until then nothing may spin.  Half a core is the bar: the stub
+    sleeps, and copying the 24 MB takes some 10 ms."""
+    run(stub, """
+        op = context(*BIG)
+        op.get_state()
+        for get in (op.get_state, lambda: op.get_gradients()[0]):
+            stub.stub_busy(400000)
+            cpu, wall = time.process_time(), time.perf_counter()
+            U = get()
+            cpu, wall = time.process_time() - cpu, time.perf_counter() - wall
+            assert right(U) and wall > 0.4 and cpu < 0.2, (cpu, wall)
+    """)
+
+
+@needs_cores
+@pytest.mark.parametrize("spare_mb", [12, 28])
+def test_plain_copy_where_threads_cannot_be_created(stub, spare_mb):
+    """Address space for the stacks of one or none of the four threads, and of two or three."""
+    run(stub, f"""
+        import resource
+        op = context(*BIG)
+        U = np.zeros(op._shape(), order="F")
+        used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+        old = resource.getrlimit(resource.RLIMIT_AS)
+        n = calls("hipMemcpyAsync")
+        resource.setrlimit(resource.RLIMIT_AS, (used + ({spare_mb} << 20), old[1]))
+        rc = _lib.lib().galx_get_state(op._h, dg._dptr(U))
+        resource.setrlimit(resource.RLIMIT_AS, old)
+        assert rc == 0 and right(U) and stub.stub_pending() == 0
+        assert calls("hipMemcpyAsync") - n in (1, 5)  # the plain copy alone, or after a first round of the slots
+    """)
