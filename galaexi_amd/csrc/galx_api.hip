@@ -773,6 +773,8 @@ static int copy_staged(galx_ctx* c, const std::vector<HostOut>& chunks, bool& co
         tell();
     }
     for (auto& t : team) t.join();
+    // the copies queued before an error write to the slots that the next call uses
+    if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);
     HIPCHK(e);
     copied = true;
     return GALX_OK;
@@ -800,8 +802,13 @@ static int copy_to_host(galx_ctx* c, std::initializer_list<HostOut> parts)
         }
         if (rc || copied) return rc;
     }
-    for (const HostOut& p : parts) HIPCHK(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    hipError_t e = hipSuccess;
+    for (const HostOut& p : parts)
+        if (e == hipSuccess) e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, c->stream);
+    // on an error too: the caller may free the arrays that the copies queued so far write to
+    const hipError_t es = hipStreamSynchronize(c->stream);
+    HIPCHK(e);
+    HIPCHK(es);
     return GALX_OK;
 }
 

@@ -111,3 +111,28 @@ def test_plain_copy_where_threads_cannot_be_created(stub, spare_mb):
         assert rc == 0 and right(U) and stub.stub_pending() == 0
         assert calls("hipMemcpyAsync") - n in (1, 5)  # the plain copy alone, or after a first round of the slots
     """)
+
+
+@needs_cores
+@pytest.mark.parametrize("call,nth", [("hipMemcpyAsync", 3), ("hipMemcpyAsync", 9), ("hipEventRecord", 2),
+                                      ("hipEventSynchronize", 1), ("hipEventSynchronize", 7)])
+def test_no_copy_outlives_a_failed_call(stub, call, nth):
+    """A copy still under way would write into the slots of the next call, or into an array the caller has freed."""
+    run(stub, f"""
+        op = context(*BIG)
+        assert right(op.get_state())
+        fail("{call}", {nth})
+        assert "stub error" in refused(op.get_state)
+        assert stub.stub_pending() == 0
+        stub.hipGetLastError()  # the runtime keeps it until it is asked
+        assert right(op.get_state()) and stub.stub_pending() == 0
+    """)
+
+
+def test_no_plain_copy_outlives_a_failed_call(stub):
+    run(stub, """
+        op = context(4, (3, 3, 3))
+        fail("hipMemcpyAsync", 2)
+        assert "stub error" in refused(op.get_gradients)
+        assert stub.stub_pending() == 0
+    """)
