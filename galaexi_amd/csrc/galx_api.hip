@@ -1125,6 +1125,7 @@ int galx_set_mesh(galx_ctx* c, int nElems, int nSides, const int* E2S, const int
 static int state_in(galx_ctx* c, const double* dSrc)
 {
     c->trajValid = false;  // a recorded trajectory no longer ends at the context state
+    c->stateSet = c->utValid = false;  // until all parts of the new state are there
     c->kZero = true;
     c->cur = 0;
     c->pref = 0.0;
@@ -1156,9 +1157,8 @@ static int state_in(galx_ctx* c, const double* dSrc)
         c->ks.trace(c->stream, c->nElems, c->dU, mesh_of(c), c->dUtr[0], gas_of(c));
     }
     HIPCHK(hipGetLastError());
-    c->stateSet = true;
-    c->utValid = false;
     HIPCHK(hipStreamSynchronize(c->stream));
+    c->stateSet = true;
     return GALX_OK;
 }
 

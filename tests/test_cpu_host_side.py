@@ -136,3 +136,21 @@ def test_no_plain_copy_outlives_a_failed_call(stub):
         assert "stub error" in refused(op.get_gradients)
         assert stub.stub_pending() == 0
     """)
+
+
+@pytest.mark.parametrize("N,precision,launch", [(3, "fp64", 1), (3, "mixed", 1), (3, "mixed", 2), (11, "fp64", 1)])
+def test_failed_set_state_leaves_no_state(stub, N, precision, launch):
+    """The state's planes and its traces, offsets and register belong together: after a call that wrote only some of them
+    there is nothing to step from."""
+    run(stub, f"""
+        op = context({N}, (2, 2, 2), "{precision}")
+        U = np.ones(op._shape(), order="F")
+        op.TimeStepByLSERKW2(0.0, 1e-3)
+        fail("hipLaunchKernel", {launch})
+        assert "stub error" in refused(op.set_state, U)
+        for call in (lambda: op.TimeStepByLSERKW2(0.0, 1e-3), lambda: op.lserk_stage(0.0, 1e-3, 1), op.get_state,
+                     op.CalcTimeStep, op.get_gradients, op.rhs_only):
+            assert "set_state first" in refused(call)
+        op.set_state(U)
+        op.TimeStepByLSERKW2(0.0, 1e-3)
+    """)
