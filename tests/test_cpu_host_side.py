@@ -150,7 +150,7 @@ def test_failed_set_state_leaves_no_state(stub, N, precision, launch):
         assert "stub error" in refused(op.set_state, U)
         for call in (lambda: op.TimeStepByLSERKW2(0.0, 1e-3), lambda: op.lserk_stage(0.0, 1e-3, 1), op.get_state,
                      op.CalcTimeStep, op.get_gradients, op.rhs_only):
-            assert "set_state first" in refused(call)
+            assert any(why in refused(call) for why in ("set_state first", "no state"))
         op.set_state(U)
         op.TimeStepByLSERKW2(0.0, 1e-3)
     """)
