@@ -1806,7 +1806,9 @@ static int adj_reverse(galx_ctx* c)
         // alternate between the context's two trace buffers, and the VJPs recompute FP64 records from the stage inputs.
         const bool keep = c->tsz == 8;
         c->ks.trace(c->stream, c->nElems, c->ckpt[seg], m, keep ? (void*)c->stageTr[0] : c->dUtr[0], gd);
-        for (int s = 0; s < n && c->stagesSeg != seg; s++)
+        const bool there = c->stagesSeg == seg;
+        c->stagesSeg = -1;  // until the launches below have gone well
+        for (int s = 0; s < n && !there; s++)
             for (int stage = 0; stage < 5; stage++) {
                 const int idx = 5 * s + stage;
                 const bool last = idx + 1 == 5 * n;
@@ -1819,8 +1821,8 @@ static int adj_reverse(galx_ctx* c)
                 const double ts = stage_time(step_time(c->trajT, c->trajDt, s0 + s), c->trajDt, stage);
                 launch_rhs(c, Stage{mRKA, RKB[stage] * c->trajDt, 1, stage == 4}, ts, Ui, Uo, tri, tro);
             }
-        c->stagesSeg = seg;
         HIPCHK(hipGetLastError());
+        c->stagesSeg = seg;
         // reverse
         for (int s = n - 1; s >= 0; s--)
             for (int stage = 4; stage >= 0; stage--) {

@@ -154,3 +154,22 @@ def test_failed_set_state_leaves_no_state(stub, N, precision, launch):
         op.set_state(U)
         op.TimeStepByLSERKW2(0.0, 1e-3)
     """)
+
+
+def test_failed_recompute_is_not_taken_for_the_stages(stub):
+    """The sweep counts the stage inputs of a segment as there once their kernels have been launched: the sweep after a failed
+    one launches what one without the failure does."""
+    run(stub, """
+        op = context(3, (2, 2, 2))
+        lam = np.ones(op._shape(), order="F")
+        op.forward_ckpt(0.0, 1e-3, 4, 2)
+        op.lserk_adjoint(lam)  # the last segment's stages come from the recorded run; it leaves those of the first one
+        n = calls("hipLaunchKernel")
+        op.lserk_adjoint(lam)
+        full = calls("hipLaunchKernel") - n
+        fail("hipLaunchKernel", 10)  # in the recompute of the last segment
+        assert "stub error" in refused(op.lserk_adjoint, lam)
+        n = calls("hipLaunchKernel")
+        op.lserk_adjoint(lam)
+        assert calls("hipLaunchKernel") - n == full
+    """)
