@@ -612,17 +612,23 @@ static GasD gas_of(galx_ctx* c)
 // the adjoint kernels and their FP64 trace records use the pressure itself (no offset)
 static GasD adj_gas_of(galx_ctx* c) { return make_gasd(c->cfg.kappa, c->cfg.R, c->cfg.mu0, c->lambda, 0.0, 0.0); }
 
-// two pinned host buffers that alternate as staging for host-to-device copies: next() returns a buffer whose
-// previous copy has finished, issued() marks the copies just enqueued from it
+// two pinned host buffers that alternate as staging for host-to-device copies, its own or the halves of `base`: next()
+// returns a buffer whose previous copy has finished, issued() marks the copies just enqueued from it
 struct Staging {
     double* p[2] = {nullptr, nullptr};
+    bool own = true;
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool busy[2] = {false, false};
     int k = 1;
-    int init(size_t bytes)
+    int init(size_t bytes, char* base)
     {
+        own = !base;
         for (int i = 0; i < 2; i++) {
-            hipError_t e = hipHostMalloc((void**)&p[i], bytes, hipHostMallocDefault);
+            hipError_t e = hipSuccess;
+            if (base)
+                p[i] = (double*)(base + i * bytes);
+            else
+                e = hipHostMalloc((void**)&p[i], bytes, hipHostMallocDefault);
             if (e != hipSuccess) {
                 p[i] = nullptr;
                 return fail(GALX_E_NOMEM, "hipHostMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
@@ -661,7 +667,7 @@ struct Staging {
                 (void)hipEventSynchronize(ev[i]);
                 (void)hipEventDestroy(ev[i]);
             }
-            if (p[i]) (void)hipHostFree(p[i]);
+            if (own && p[i]) (void)hipHostFree(p[i]);
         }
     }
 };
@@ -682,6 +688,13 @@ struct HostOut {
     size_t bytes;
 };
 static constexpr size_t OUT_MIN = 2 * OUT_CHUNK;
+
+// Pinned chunks of the context, allocated by galx_set_mesh for a mesh whose results can be that large (the gradients of
+// five variables are the largest): the geometry goes through them, and they stay for the results.  Allocated at the first
+// large result, they took 1.5 ms of it: ms for the first state of a context, in plain copies, with the chunks allocated
+// there and as now, N = 7 on MI355X: 6^3 elements 0.36, 2.0, 0.41; 8^3 0.9, 1.9, 0.8; 16^3 7.9, 4.5, 3.2.  galx_set_mesh
+// itself, with two pinned buffers of up to 66 MB before: 8^3 20 -> 7 ms, 16^3 70 -> 13.
+static bool large_results(long nDOF) { return 15 * nDOF * sizeof(double) >= OUT_MIN; }
 
 static bool out_staging(galx_ctx* c)
 {
@@ -788,7 +801,7 @@ static int copy_to_host(galx_ctx* c, std::initializer_list<HostOut> parts)
         bytes += p.bytes;
         staged = staged && pageable(p.dst);
     }
-    if (staged && bytes >= OUT_MIN && out_staging(c)) {
+    if (staged && bytes >= OUT_MIN && c->hStage) {
         bool copied = false;
         int rc = GALX_OK;
         try {
@@ -836,6 +849,8 @@ static void free_mesh(galx_ctx* c)
         dfree(*p);
         *p = nullptr;
     }
+    if (c->hStage) (void)hipHostFree(c->hStage);
+    c->hStage = nullptr;
 }
 
 // device buffers of galx_set_mesh and their contents; on failure the caller frees what was allocated
@@ -875,10 +890,12 @@ static int set_mesh_device(galx_ctx* c, int nElems, int nSides, const std::vecto
     // geometry into element / side planes, in chunks through two pinned staging buffers: the host fills one while
     // the copy of the other runs.  The surface-node copy of the element geometry (k_lift's metrics) comes from the
     // same planes.
-    const long chunkE = std::min(1024, nElems), chunkS = std::min(4096, nSides);  // at most 66 MB a buffer at N=7
-    const size_t stageB = std::max(10 * chunkE * (n3 + ns), 10 * chunkS * n2) * sizeof(double);
+    const size_t perE = 10L * (n3 + ns) * sizeof(double), perS = 10L * n2 * sizeof(double);
+    if (large_results(nDOF) && !out_staging(c)) return fail(GALX_E_NOMEM, "no pinned memory for staging");
+    const size_t stageB = c->hStage ? OUT_SLOTS * OUT_CHUNK / 2 : std::max(nElems * perE, nSides * perS);
+    const long chunkE = std::min((long)nElems, (long)(stageB / perE)), chunkS = std::min((long)nSides, (long)(stageB / perS));
     Staging stg;
-    if ((rc = stg.init(stageB))) return rc;
+    if ((rc = stg.init(stageB, c->hStage))) return rc;
     std::vector<int> snode(ns);
     for (int t = 0; t < ns; t++) snode[t] = surface_node_of(c->N, t);
     for (long e0 = 0; e0 < nElems; e0 += chunkE) {

@@ -173,3 +173,37 @@ def test_failed_recompute_is_not_taken_for_the_stages(stub):
         op.lserk_adjoint(lam)
         assert calls("hipLaunchKernel") - n == full
     """)
+
+
+@needs_cores
+def test_first_results_allocate_nothing_but_their_scratch(stub):
+    """The pinned chunks are those that galx_set_mesh staged the geometry through: pinning them at the first result took
+    longer than the chunks save there."""
+    run(stub, """
+        for N, nel in (BIG, (7, (9, 5, 4)), (11, (4, 3, 2))):
+            op = context(N, nel)
+            pinned, copies = calls("hipHostMalloc"), calls("hipMemcpyAsync")
+            g = op.get_gradients(5)
+            assert calls("hipHostMalloc") == pinned and calls("hipMemcpyAsync") - copies >= 3
+            n = g[0].size
+            assert all(np.array_equal(a.ravel(order="F"), np.arange(d * n, (d + 1) * n)) for d, a in enumerate(g))
+            op.close()
+        n = calls("hipHostMalloc")
+        context(7, (3, 3, 3)).close()  # its largest result stays below 4 MiB: two buffers for the geometry, dt's two doubles
+        assert calls("hipHostMalloc") - n == 3
+    """)
+
+
+def test_failed_set_mesh_leaves_nothing_pinned(stub):
+    run(stub, """
+        op = dg.DGOperator(7, form="split", riemann="lf", mu0=1e-3, R=1.0)
+        m = M.box_mesh((9, 5, 4), 7, lo=(-1.0,) * 3, hi=(1.0,) * 3)
+        for call, nth in (("hipHostMalloc", 1), ("hipMemcpyAsync", 1), ("hipMemcpyAsync", 7), ("hipEventRecord", 2)):
+            held = calls("hipHostMalloc") - calls("hipHostFree")
+            fail(call, nth)
+            assert "stub error" in refused(op.set_mesh, m) or call == "hipHostMalloc"
+            stub.hipGetLastError()
+            assert stub.stub_pending() == 0
+            assert calls("hipHostMalloc") - calls("hipHostFree") - (call == "hipHostMalloc") == held
+        op.set_mesh(m)
+    """)
