@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgalx.so")
 
-# FP64: N <= 9 one volume node per thread, N = 10..13 the high-order kernels (the degrees of the reference's
+# FP64: N <= 9 one volume node per thread, N = 10..13 the plane kernels (the degrees of the reference's
 # p-convergence check, regressioncheck/checks/convtest/p_3D); the discrete adjoint for N <= 8
 DEFAULT_FP64 = tuple(range(1, 14))
 DEFAULT_MIXED = (3, 5, 7)

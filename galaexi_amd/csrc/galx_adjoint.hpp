@@ -348,10 +348,10 @@ __global__ void __launch_bounds__(Dm<N>::block)
 // Bound by latency at the waves in flight, whose number the registers set at N = 5 and 7 and the LDS elsewhere.  The
 // split phase comes last and the faces return their adjoint in primitive form, so that next to nothing of
 // the primitive adjoint is held through the lifting and the faces, and one transposed Jacobian per node takes it all.
-// With the split phase first and a Jacobian per face node the kernel needed 142 registers at N = 5 (now 125: four
-// instead of three workgroups per CU) and spilled 60 bytes per lane at N = 7 (now 20).  us per stage of the reverse
-// sweep before -> now: N = 3, 24^3 elements 242 -> 219; N = 4, 20^3 257 -> 244; N = 5, 16^3 205 -> 181; N = 6, 14^3
-// 305 -> 283; N = 7, 16^3 461 -> 421; N = 8, 12^3 328 -> 317.
+// With the split phase first and a Jacobian per face node the kernel needed 142 registers at N = 5 (now 124: four
+// instead of three workgroups per CU) and spilled 60 bytes per lane at N = 7 (now 20).  us of the kernel in a reverse sweep
+// (kernel trace) before -> now: N = 3, 24^3 elements 202 -> 170; N = 4, 20^3 214 -> 184; N = 5, 16^3 172 -> 151; N = 6,
+// 14^3 274 -> 257; N = 7, 16^3 394 -> 353; N = 8, 12^3 279 -> 274; the k_adj_pre before it takes 42 (N = 5) to 89 (N = 7).
 // LDS: one work array reused by the phases, mu = -sJ*lam, the own stress at the face nodes and the matrices
 // (76.5 KB at N=7: two workgroups per CU, with AdjWaves capping the registers to match).
 // ---------------------------------------------------------------------------------------------------------

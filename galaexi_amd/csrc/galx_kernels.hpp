@@ -33,6 +33,8 @@
 
 namespace galx {
 
+constexpr int CUS = 256;  // compute units of an MI355X: the lines of the dispatch rules count workgroups per CU
+
 // one workgroup per element: n^3 threads rounded up to whole waves, at most 1024 (N <= 9 gives every volume node a
 // thread of its own; for N >= 10 the plane kernels take the stage, and the kernels here that run for every degree loop
 // their 1024 threads over the nodes)
@@ -85,12 +87,14 @@ struct Pack {
 // 64 and 128 threads of the volume nodes need two.  us on MI355X, before -> after:
 //   k_lift in FP64 always runs with them: N = 3 9.1 -> 8.0 at 8^3 elements, 21.0 -> 20.4 at 16^3, 86.5 -> 85.3 at 28^3;
 //   N = 4 11.8 -> 10.9 at 9^3, 31.1 -> 29.7 at 16^3.  Mixed 8.5 -> 7.3 at 8^3, 14.4 -> 13.1 at 16^3, but 47.8 -> 50.3 at
-//   28^3: up to the 16 workgroups per CU that fit beside each other.
+//   28^3: up to the 16 workgroups per CU that fit beside each other (a stage, k_rhs included, 15.1 -> 13.9 at 8^3, 32.1 ->
+//   31.2 at 16^3).
 //   k_rhs does on meshes that do not fill the chip: its face task is a longer part of the workgroup's serial chain, but in
 //   the other phases the added wave only waits, and holds registers that another workgroup could use.  N = 3 weak Roe 13.6
 //   -> 11.7 at 8^3, 18.3 -> 16.2 at 11^3, split RoeEntropyFix 22.8 -> 25.2 at 12^3: the line is six workgroups per CU, all
-//   that fit beside each other.  N = 4 split LF 19.0 -> 17.1 at 8^3, 50.3 -> 47.9 at 14^3, weak Roe 59.2 -> 60.4 at 16^3:
-//   twelve per CU.
+//   that fit beside each other; mixed, up to the same line, a stage of split LF 15.3 -> 13.9 at 8^3, 19.0 -> 17.5 at 11^3,
+//   weak Roe 14.4 -> 13.4 and 18.5 -> 17.1.  N = 4 split LF 19.0 -> 17.1 at 8^3, 50.3 -> 47.9 at 14^3, weak Roe 59.2 ->
+//   60.4 at 16^3: twelve per CU.
 template <int N>
 struct FaceBlock {
     static constexpr bool wider = N == 3 || N == 4;
@@ -98,9 +102,9 @@ struct FaceBlock {
     template <typename T>
     static bool lift(int nElems)
     {
-        return wider && (sizeof(T) == 8 || nElems <= 16 * 256);
+        return wider && (sizeof(T) == 8 || nElems <= 16 * CUS);
     }
-    static bool rhs(int nElems) { return wider && nElems <= (N == 3 ? 6 : 12) * 256; }
+    static bool rhs(int nElems) { return wider && nElems <= (N == 3 ? 6 : 12) * CUS; }
 };
 
 // nodes on the element surface, n^3 - (n-2)^3 of them
@@ -1071,12 +1075,13 @@ __global__ void __launch_bounds__(Dm<N>::block)
 // The lean order of the FP64 form, for fewer live registers and less LDS: the lean gradient; in the split form the viscous
 // terms of all directions before the pairs (the stress tensor dies before the pairs, whose sum then starts from the
 // viscous one, and 9 instead of 13 node planes share the work region); the viscous-flux traces loaded after the Riemann
-// flux.  Registers without a cap at N = 7 (split): LF 126 (capped, 128) -> 102, Roe 150 -> 116, RoeEntropyFix 142 -> 120,
+// flux.  Registers without a cap at N = 7 (split): LF 126 (capped, 128) -> 102, Roe 150 -> 118, RoeEntropyFix 142 -> 122,
 // so that every solver runs two 8-wave workgroups per CU without spilling; LDS at N = 7 71.7 -> 55.3, at N = 8
-// 97 -> 74 KB (two workgroups per CU).  k_rhs on MI355X, FP64, before -> after:
-//   split RoeEntropyFix N = 7, 20^3 elements   645 -> 443 us     split LF N = 8, 16^3   441 -> 344 us
-//   split LF N = 6, 16^3                       201 -> 182 us     split LF N = 5, 24^3   315 -> 303 us
-//   weak Roe N = 5, 20^3                       220 -> 187 us
+// 97 -> 74 KB (two workgroups per CU).  k_rhs on MI355X, FP64, HIP events, before -> now (the register's reads and stores
+// that Stage leaves out included):
+//   split RoeEntropyFix N = 7, 20^3 elements   641 -> 405 us     split LF N = 8, 16^3   435 -> 305 us
+//   split LF N = 6, 16^3                       193 -> 169 us     split LF N = 5, 24^3   293 -> 279 us
+//   weak Roe N = 5, 20^3                       206 -> 174 us     split Roe N = 7, 20^3  424 -> 401 us
 // Split LF at N = 7 keeps the other order, with the lifting's line derivatives on the matrix cores (node_gradient_mfma,
 // no registers to spare for Roe beside it): it runs at two workgroups per CU either way, and the stage, the k_lift behind
 // it included, measured 0.5 to 0.8 % faster.
@@ -1128,7 +1133,7 @@ __device__ __forceinline__ void face_flux(const T* tro, const T* trn, T* fv, con
 // minimum waves per SIMD for k_rhs.  FP64: the compiler's choice (at most 128 registers in the lean order) except where
 // LF, the lightest solver, fits one workgroup more without spilling or with little of it: 5 waves at N = 5 (five 4-wave
 // workgroups per CU, 99 against 103 us on 16^3 elements) and at N = 6 in the split form (three 6-wave ones), 6 at N = 8 in
-// the split form (two 12-wave ones, 80 registers with 6 spilled: 344 against 445 us on 16^3).  The Roe solvers spill
+// the split form (two 12-wave ones, 80 registers with 4 spilled: 344 against 445 us on 16^3).  The Roe solvers spill
 // under the same caps and lose (N = 6 Roe 218 -> 251 us).  Mixed: 6 lets three 512-thread workgroups share a CU at N = 7
 // (80 registers, which its LDS share allows); the entropy-fixed Roe solver and the small blocks of N < 5 keep the
 // compiler's choice.

@@ -10,15 +10,25 @@
 //                 workspace, the face fluxes, -sJ, the register update and the next traces.
 // The gradients are formed once per stage, where k_lift and k_rhs form the surface nodes' twice; the price is the
 // workspace, 9 (split) or 10 (weak) values per node written and read once, and each column read by every plane.
-// On small meshes both kernels are bound by the latency of one workgroup's instruction stream (about 2500 instructions
-// a wave, FP64 at one wave per SIMD), not by bytes: loads issued ahead of the state changed nothing and cost spills.
-// Measured on MI355X, FP64, both stage kernels together, against one workgroup per element (k_lift + k_rhs for N <= 9;
-// for N >= 10 kernels with all work arrays in HBM that these replaced):
-//   N = 11, 2^3 elements, split, RoeEntropyFix   303 -> 24 us
-//   N = 9, split, LF: 2^3 44 -> 24, 4^3 45 -> 32, 5^3 48 -> 43, 6^3 52 -> 65 us
-//   N = 7, split, LF: 2^3 30 -> 21, 4^3 30 -> 24, 5^3 32 -> 28, 6^3 34 -> 36 us
-//   N = 4, split, LF: 2^3 23 -> 20, 4^3 23 -> 19, 6^3 24 -> 22, 8^3 29 -> 27 us
-// and on meshes that fill the chip they lose: N = 8, 12^3 247 -> 275, N = 9, 12^3 347 -> 416 us.
+// On small meshes both kernels are bound by the latency of one workgroup's instruction stream, not by bytes: k_vol_plane
+// issues 2272 VALU and 291 LDS instructions a wave at N = 11 (2^3 elements, 15.3 us, 0.3 TB/s, VALU busy 4 %, occupancy
+// 2 %), 1666 and 220 at N = 7 (4^3, 13.2 us, 0.8 TB/s, 6 %, 3 %); loads issued ahead of the state changed nothing and cost
+// spills.  Measured on MI355X, FP64, us per stage of a run, launches included, with one workgroup per element (k_lift +
+// k_rhs) and with planes, split LF, weak Roe and split RoeEntropyFix:
+//   N = 4: 2^3 16.6 -> 16.2, 15.3 -> 15.5, 17.1 -> 17.5; 4^3 16.7 -> 15.5, 15.3 -> 15.1, 17.1 -> 16.9;
+//          5^3 16.9 -> 17.3, 15.6 -> 16.7, 17.4 -> 18.5; 6^3 17.5 -> 18.0, 16.0 -> 17.1, 17.9 -> 19.2
+//   N = 5: 2^3 19.8 -> 16.4, 17.1 -> 15.0, 20.3 -> 17.5; 5^3 20.4 -> 19.7, 17.6 -> 17.2, 20.8 -> 20.6;
+//          6^3 21.1 -> 22.0, 18.5 -> 20.5, 21.6 -> 23.3
+//   N = 6: 4^3 22.6 -> 18.4, 19.9 -> 17.0, 23.7 -> 19.6; 5^3 23.5 -> 21.7, 20.7 -> 20.5, 24.6 -> 22.7;
+//          6^3 24.9 -> 24.3, 21.9 -> 23.1, 25.9 -> 26.1
+//   N = 7: 2^3 25.4 -> 17.5, 22.2 -> 16.1, 26.8 -> 18.7; 5^3 26.9 -> 23.0, 23.7 -> 21.4, 28.5 -> 24.5;
+//          6^3 28.4 -> 30.0, 25.0 -> 28.3, 29.7 -> 32.6
+//   N = 8: 4^3 33.1 -> 22.8, 27.0 -> 20.6, 32.7 -> 23.8; 5^3 35.0 -> 30.2, 28.4 -> 27.3, 34.2 -> 31.7;
+//          6^3 37.3 -> 39.4, 30.1 -> 35.6, 36.4 -> 40.7
+//   N = 9: 2^3 37.6 -> 20.1, 30.9 -> 17.3, 39.2 -> 24.6; 4^3 38.3 -> 26.4, 31.6 -> 22.6, 39.9 -> 30.6;
+//          5^3 40.1 -> 35.8, 33.3 -> 30.3, 41.8 -> 44.3; 6^3 43.0 -> 55.2, 35.6 -> 47.6, 44.5 -> 74.2
+// On meshes that fill the chip they lose (both kernels: N = 8, 12^3 247 -> 275, N = 9, 12^3 347 -> 416 us).  For N >= 10
+// they replaced kernels with all work arrays in HBM (N = 11, 2^3, split, RoeEntropyFix 303 -> 24 us).
 #pragma once
 #include "galx_kernels.hpp"
 
@@ -31,21 +41,24 @@ namespace galx {
 template <int N>
 struct Pl {
     static constexpr int n = N + 1, n2 = n * n, n3 = n2 * n;
-    // planes per workgroup: as many as fill its last wave where one plane leaves a third of the lanes idle (N = 4: 50 of
-    // 64 lanes, N = 8: 243 of 256; at N = 8 one plane measured 29 against 27 us on 4^3 elements)
+    // planes per workgroup: one plane is 25 of 64 lanes at N = 4 and 81 of 128 at N = 8, two and three are 50 of 64 and
+    // 243 of 256 (at N = 8 one plane measured 29 against 27 us on 4^3 elements).  N = 5, 36 of 64 lanes, has been measured
+    // with one plane only; the other degrees fill three quarters of their lanes or more
     static constexpr int planes = N == 4 ? 2 : (N == 8 ? 3 : 1);
     static constexpr int block = (planes * n2 + 63) / 64 * 64;
     static constexpr int groups = (n + planes - 1) / planes;  // workgroups per element
     static constexpr int ws = 10 * n3;  // workspace values per element: [5] volume terms, [5] contravariant flux f_3
 };
 
-// FP64 meshes of at most four planes a CU (256 CUs) take the plane kernels from N = 4 on: the line lies where the two
-// forms cross (see the figures above: 5^3 to 6^3 elements at N = 7 and 9).  The mixed form keeps its one-element kernels
-// and with them its FP32 rounding.
+// FP64 meshes of at most four planes a CU take the plane kernels from N = 4 on: one line for all degrees, near which the two
+// forms cross (see the figures above).  It is not each degree's own: the planes still win beyond it at N = 8 and 9 (5^3
+// elements, up to 14 %, but not with RoeEntropyFix at N = 9), and lose up to 7 % below it at N = 4 (5^3).  The mixed form
+// keeps its one-element kernels and with them its FP32 rounding; it takes the planes from N = 10 on, in a library built for
+// such mixed degrees (Ut at N = 11 5.5e-6 split LF, 3.8e-6 weak Roe from the FP64 oracle).
 template <int N, typename T>
 __host__ constexpr bool use_planes(int nElems)
 {
-    return N >= GALX_PLANE_DEGREE || (sizeof(T) == 8 && N >= 4 && (long)nElems * (N + 1) <= 1024);
+    return N >= GALX_PLANE_DEGREE || (sizeof(T) == 8 && N >= 4 && (long)nElems * (N + 1) <= 4 * CUS);
 }
 
 // workgroups are dealt to the 8 XCDs in turn: workgroup x takes block (x % 8) * per + x / 8 of `count` blocks, so that
@@ -253,9 +266,10 @@ __global__ void __launch_bounds__(Pl<N>::block, 4)
         }
     }
     __syncthreads();
-    // along k: the node's column from memory, for the derivative and the split pairs.  The diagonal pairs stay in on all
-    // lines, as VolInt_splitForm_Kernel has them: DVolSurf(a,a), zero up to rounding, is the residue that makes the
-    // rounded derivative matrix exact on constants (without it the N = 11 step is twice as far from the FP64 result).
+    // along k: the node's column from memory, for the derivative and the split pairs.  The diagonal pairs, which k_rhs
+    // leaves out, stay in on all lines, as VolInt_splitForm_Kernel has them: DVolSurf(a,a), zero up to rounding, is the
+    // residue that makes the rounded derivative matrix exact on constants (without it the N = 11 step is twice as far from
+    // the FP64 result).
     T gze[4] = {0, 0, 0, 0}, tmp[5] = {0, 0, 0, 0, 0};
     if (nd.active) {
         const T* gk = GeoOf<T>::geo(mesh) + (long)e * 10 * n3 + 6 * n3 + r;
