@@ -681,7 +681,7 @@ struct Staging {
 // threads no faster, 8 slots 16 % faster at 84 MB only, for a longer first call.  The threads sleep until the first chunk
 // arrives, i.e. until the work queued before the call has ended (a host-form reverse sweep of 22 ms took 98 ms of processor
 // time while they spun there, and takes 22), and spin for at most OUT_SPIN_US after that.  Pinned destinations and small
-// ones keep the plain copy, and so does a host that has no memory or threads to give.
+// ones keep the plain copy, and so does a host that has few cores or no threads to give.
 struct HostOut {
     double* dst;
     const double* src;
